@@ -248,3 +248,12 @@ def test_synth_full_1024_chunk(hip):
     into two chunks of near-equal length (neither a multiple of the other),
     each token the step's bits."""
     compare_models(BASE, 14, 8, True, 1024, [1025], n_after=3, max_ctx=1040)
+
+
+@pytest.mark.parametrize("heads,kv,hd", [(8, 8, 32), (8, 2, 96), (16, 1, 128), (20, 4, 64)])
+def test_attention_row_tiles(hip, heads, kv, hd):
+    """Row tiles of the attention launches (32 score rows, 16 P.V rows, 64
+    positions, groups of 16 positions): part tiles, one row more than a tile,
+    tokens of one tile at positions on both sides of a group's end."""
+    compare_models(dict(BASE, n_heads=heads, n_kv_heads=kv, head_dim=hd), 14, 8, True, 0, [15, 1, 17, 31, 33, 2, 64],
+                   n_after=2)

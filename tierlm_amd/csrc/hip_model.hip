@@ -945,22 +945,35 @@ __global__ __launch_bounds__(NT) void k_attn_merge(const float *__restrict__ par
  * k_pf_prep: a group per token: q-norm + RoPE of every query head in place,
  *   k-norm + RoPE of every key head (norm_rope16, the decode's code), the key
  *   and value appended to the cache at the token's position.
- * k_pf_scores: a group per (key head, PF_TOK tokens, 64 positions): lane =
- *   position with its key row in registers, wave = token, HB query heads of
- *   the key head at a time from LDS; each score is the dot in ascending i,
- *   scaled after the dot (the decode's expression).
+ * k_pf_scores: a wave per (key head, PF_SROWS rows, 64 positions), a row being
+ *   one query head of one token; each score is the dot in ascending i, scaled
+ *   after the dot (the decode's expression).
  * k_pf_softmax: a group per (token, query head): the decode P.V launch's
  *   softmax with its thread mapping and reduction trees (the maximum, e_t,
  *   their double sum, inv); p_t = e_t * inv replaces the score.
- * k_pf_pv: a group per (key head, 64-element slab, PF_TOK tokens): lane =
- *   element, wave = token, one chain per query head (HB at a time), out +=
- *   p_t * v_t[i] over ascending t up to the token's position (the rounded
- *   product, then the add), the probabilities staged in LDS PF_PCH positions
- *   at a time.  Products past the position are never added (adding +0 would
- *   leave the chain unchanged, as in the decode ring).
+ * k_pf_pv: a wave per (key head, 64-element slab, PF_VROWS rows), out +=
+ *   p_t * v_t[i] over ascending t up to the row's position (the rounded
+ *   product, then the add); a group's waves share their rows' probabilities.
+ * The dots and P.V are chains of a rounded product and a rounded add, and an
+ * fma would round once.  The products of one i (one t) over a tile are an
+ * outer product: v_mfma_f32 with K = 1 and C = 0 gives each of them with the
+ * rounding of v_mul_f32 (subnormals and signed zeros included), 2048 in 64
+ * lanes, and the VALU only adds.  Operands come from L1 / L2 straight into
+ * registers, 16 elements (positions) ahead of their use, so no LDS read sits
+ * between the adds: with the products on the VALU and the query values or
+ * probabilities broadcast from LDS both launches waited for LDS.  At 682
+ * tokens behind 1365 positions, 32 heads of 128 (4.8 G products each): scores
+ * 381 -> 211 us, P.V 387 -> 195 us (24.5 G products / ms; a loop of the two
+ * instructions alone runs at 34.5, v_mul + v_add at 26.4).  Bound: VALU issue
+ * of the adds and the matrix pipe, which do not fully overlap.  P.V takes 16
+ * rows a wave (the score launch 32): its chains are as long as the context, so
+ * waves are what is short.
  * Score rows: [token][query head][SL] floats, SL the capacity rounded up to 4. */
-constexpr int PF_TOK = 4;     /* tokens per group, a wave each */
-constexpr int PF_PCH = 256;   /* positions per staged chunk of probabilities */
+constexpr int PF_SROWS = 32;  /* rows per wave of the score launch */
+constexpr int PF_VROWS = 16;  /* rows per wave of the P.V launch */
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
+__host__ __device__ constexpr int pf_slabs(int hd) { return (hd + 63) / 64; }
 
 template <int HD>
 __global__ __launch_bounds__(NT) void k_pf_prep(float *__restrict__ q, const float *__restrict__ kx,
@@ -999,50 +1012,62 @@ __global__ __launch_bounds__(NT) void k_pf_prep(float *__restrict__ q, const flo
     }
 }
 
-template <int HD, int HB>
+/* the launch's rows of one key head: row r is query head r % R of token r / R */
+template <int HD>
 __global__ __launch_bounds__(NT) void k_pf_scores(const float *__restrict__ q, const float *__restrict__ kc,
                                                   float *__restrict__ scores, int H, int KV, int max_ctx, int p0,
                                                   int ntok, int SL) {
-    constexpr int H4 = HD / 4;
-    __shared__ __align__(16) f32x4 s_q[PF_TOK][HB][H4];
-    const int R = H / KV, kvh = blockIdx.z, tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int t0 = (int)blockIdx.y * PF_TOK, u0 = (int)blockIdx.x * 64;
-    const int tlast = min(t0 + PF_TOK, ntok) - 1;
-    if (u0 > p0 + tlast) return;   /* uniform: no token of the group reaches these positions */
-    const int t = t0 + wave, P = t < ntok ? p0 + t : -1, u = u0 + lane;
-    /* the lane's key row (positions past the group's last are clamped, never stored) */
-    const f32x4 *K4 = (const f32x4 *)(kc + ((size_t)kvh * max_ctx + min(u, p0 + tlast)) * HD);
-    f32x4 kr[H4];
+    constexpr int NC = HD / 16;   /* chunks of 16 elements, an even number */
+    static_assert(HD % 32 == 0, "chunks go in pairs");
+    const int R = H / KV, kvh = blockIdx.z, lane = threadIdx.x & 63, nrows = ntok * R;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = ((int)blockIdx.y * (NT / 64) + wave) * PF_SROWS, u0 = (int)blockIdx.x * 64;
+    const int plast = p0 + min(r0 + PF_SROWS - 1, nrows - 1) / R;
+    if (r0 >= nrows || u0 > plast) return;   /* uniform over the wave; the kernel has no barrier */
+    /* rows past the launch's last and positions past the wave's last are clamped, never stored */
+    const int ra = min(r0 + (lane & 31), nrows - 1);
+    const f32x4 *A4 = (const f32x4 *)(q + ((size_t)(ra / R) * H + kvh * R + ra % R) * HD);
+    const f32x4 *B4 = (const f32x4 *)(kc + ((size_t)kvh * max_ctx + min(u0 + lane, plast)) * HD);
+    f32x4 a[2][4], b[2][4];
+    auto load = [&](int s, int c) {
 #pragma unroll
-    for (int i4 = 0; i4 < H4; i4++) kr[i4] = K4[i4];
-    const float scale = 1.0f / sqrtf((float)HD);
-    for (int hb = 0; hb < R; hb += HB) {   /* uniform */
-        if (hb > 0) __syncthreads();       /* the previous heads are read */
-        for (int idx = tid; idx < PF_TOK * HB * H4; idx += NT) {
-            const int tk = idx / (HB * H4), j = (idx / H4) % HB, i4 = idx % H4;
-            const int tt = min(t0 + tk, ntok - 1);
-            s_q[tk][j][i4] = ((const f32x4 *)(q + ((size_t)tt * H + kvh * R + hb + j) * HD))[i4];
+        for (int k = 0; k < 4; k++) {
+            a[s][k] = A4[4 * c + k];
+            b[s][k] = B4[4 * c + k];
         }
-        __syncthreads();
-        float acc[HB];
+    };
+    float acc[32];
 #pragma unroll
-        for (int j = 0; j < HB; j++) acc[j] = 0.0f;
+    for (int v = 0; v < 32; v++) acc[v] = 0.0f;
+    load(0, 0);
+    v32f pr = __builtin_amdgcn_mfma_f32_32x32x1f32(a[0][0].x, b[0][0].x, v32f{}, 0, 0, 0);
+    for (int c = 0; c < NC; c += 2) {
 #pragma unroll
-        for (int i4 = 0; i4 < H4; i4++) {   /* whole: the key row stays in registers */
-            const f32x4 b = kr[i4];
+        for (int s = 0; s < 2; s++) {
+            load(s ^ 1, min(c + s + 1, NC - 1));
 #pragma unroll
-            for (int j = 0; j < HB; j++) {
-                const f32x4 a = s_q[wave][j][i4];
-                acc[j] += a.x * b.x;
-                acc[j] += a.y * b.y;
-                acc[j] += a.z * b.z;
-                acc[j] += a.w * b.w;
+            for (int e = 0; e < 16; e++) {   /* element e + 1's products are issued before element e's are added */
+                const f32x4 an = e < 15 ? a[s][(e + 1) >> 2] : a[s ^ 1][0];
+                const f32x4 bn = e < 15 ? b[s][(e + 1) >> 2] : b[s ^ 1][0];
+                const v32f nx = __builtin_amdgcn_mfma_f32_32x32x1f32(an[(e + 1) & 3], bn[(e + 1) & 3], v32f{}, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 32; v++) acc[v] += pr[v];
+                pr = nx;
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);    /* one MFMA, */
+                __builtin_amdgcn_sched_group_barrier(0x2, 32, 0);   /* then the adds */
             }
         }
-        if (u <= P) {
+    }
+    const float scale = 1.0f / sqrtf((float)HD);
 #pragma unroll
-            for (int j = 0; j < HB; j++) scores[((size_t)t * H + kvh * R + hb + j) * SL + u] = acc[j] * scale;
+    for (int v = 0; v < 16; v++) {
+        const int r = r0 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3), t = r / R;
+        if (r >= nrows) continue;
+        float *S = scores + ((size_t)t * H + kvh * R + r % R) * SL;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int u = u0 + 32 * h + (lane & 31);
+            if (u <= p0 + t) S[u] = acc[16 * h + v] * scale;
         }
     }
 }
@@ -1108,68 +1133,74 @@ __global__ __launch_bounds__(NT) void k_pf_softmax(float *__restrict__ scores, i
     }
 }
 
-template <int HD, int HB>
+template <int HD>
 __global__ __launch_bounds__(NT) void k_pf_pv(const float *__restrict__ scores, const float *__restrict__ vc,
                                               float *__restrict__ att, int H, int KV, int max_ctx, int p0, int ntok,
                                               int SL) {
-    constexpr int NWC = (HD + 63) / 64, PQ = PF_PCH / 4;
-    __shared__ __align__(16) f32x4 s_p[PF_TOK][HB][PQ];
-    const int R = H / KV, kvh = (int)blockIdx.x / NWC, slab = (int)blockIdx.x % NWC;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int t0 = (int)blockIdx.y * PF_TOK, tlast = min(t0 + PF_TOK, ntok) - 1, pmax = p0 + tlast;
-    const int t = t0 + wave, P = t < ntok ? p0 + t : -1, ic = 64 * slab + lane;
+    constexpr int NWC = pf_slabs(HD), RT = NT / 64 / NWC;   /* slabs, row tiles of a group */
+    const int R = H / KV, kvh = blockIdx.x, lane = threadIdx.x & 63, nrows = ntok * R;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), slab = wave % NWC;
+    const int r0 = ((int)(gridDim.y - 1 - blockIdx.y) * RT + wave / NWC) * PF_VROWS;   /* the longest rows first */
+    if (r0 >= nrows) return;   /* uniform over the wave; the kernel has no barrier */
+    const int ra = min(r0 + (lane & 15), nrows - 1);   /* rows past the last are clamped, never stored */
+    const f32x4 *A4 = (const f32x4 *)(scores + ((size_t)(ra / R) * H + kvh * R + ra % R) * SL);
     const char *vbase = (const char *)(vc + (size_t)kvh * att_vstride(max_ctx, HD));
-    const uint32_t lane_off = (uint32_t)min(ic, HD - 1) * 16u;   /* element ic's 16 bytes of a tile */
+    const uint32_t lane_off = (uint32_t)min(64 * slab + lane, HD - 1) * 16u;   /* the element's 16 bytes of a tile */
     auto vtile = [&](int tq) { return *(const f32x4 *)(vbase + (size_t)tq * (HD * 16) + lane_off); };
-    for (int hb = 0; hb < R; hb += HB) {   /* uniform */
-        float acc[HB];
+    f32x4 a[2][4], b[2][4];
+    auto load = [&](int s, int g) {   /* positions 16 g .. 16 g + 15 */
 #pragma unroll
-        for (int j = 0; j < HB; j++) acc[j] = 0.0f;
-        for (int c0 = 0; c0 <= pmax; c0 += PF_PCH) {   /* uniform */
-            __syncthreads();   /* the previous chunk is read */
-            for (int idx = tid; idx < PF_TOK * HB * PQ; idx += NT) {
-                const int tk = idx / (HB * PQ), j = (idx / PQ) % HB, u4 = idx % PQ;
-                const int tt = t0 + tk, uu = c0 + 4 * u4;
-                f32x4 pv = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (tt <= tlast && uu <= p0 + tt)   /* row tt holds positions 0 .. p0 + tt (within SL) */
-                    pv = *(const f32x4 *)(scores + ((size_t)tt * H + kvh * R + hb + j) * SL + uu);
-                s_p[tk][j][u4] = pv;
-            }
-            __syncthreads();
-            const int ue = min(P, c0 + PF_PCH - 1);   /* the wave's last position in the chunk */
-            int u = c0;
-            for (; u + 15 <= ue; u += 16) {
-                f32x4 vt[4];
-#pragma unroll
-                for (int k = 0; k < 4; k++) vt[k] = vtile((u >> 2) + k);
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-#pragma unroll
-                    for (int j = 0; j < HB; j++) {
-                        const f32x4 pp = s_p[wave][j][((u - c0) >> 2) + k];
-                        acc[j] += pp.x * vt[k].x;
-                        acc[j] += pp.y * vt[k].y;
-                        acc[j] += pp.z * vt[k].z;
-                        acc[j] += pp.w * vt[k].w;
-                    }
-                }
-            }
-            for (; u <= ue; u += 4) {   /* the last positions, up to ue */
-                const f32x4 vt = vtile(u >> 2);
-#pragma unroll
-                for (int j = 0; j < HB; j++) {
-                    const f32x4 pp = s_p[wave][j][(u - c0) >> 2];
-                    acc[j] += pp.x * vt.x;
-                    if (u + 1 <= ue) acc[j] += pp.y * vt.y;
-                    if (u + 2 <= ue) acc[j] += pp.z * vt.z;
-                    if (u + 3 <= ue) acc[j] += pp.w * vt.w;
-                }
-            }
+        for (int k = 0; k < 4; k++) {
+            a[s][k] = A4[4 * g + k];
+            b[s][k] = vtile(4 * g + k);
         }
-        if (t < ntok && ic < HD) {
+    };
+    float acc[16];
 #pragma unroll
-            for (int j = 0; j < HB; j++) att[((size_t)t * H + kvh * R + hb + j) * HD + ic] = acc[j];
+    for (int v = 0; v < 16; v++) acc[v] = 0.0f;
+    /* whole groups of 16 positions that every row of the tile attends to */
+    const int ng = (p0 + r0 / R + 1) / 16;
+    if (ng > 0) {
+        load(0, 0);
+        v16f pr = __builtin_amdgcn_mfma_f32_16x16x1f32(a[0][0].x, b[0][0].x, v16f{}, 0, 0, 0);
+        auto group = [&](int s, int next) {
+            load(s ^ 1, min(next, ng - 1));
+#pragma unroll
+            for (int e = 0; e < 16; e++) {   /* position e + 1's products are issued before position e's are added */
+                const f32x4 an = e < 15 ? a[s][(e + 1) >> 2] : a[s ^ 1][0];
+                const f32x4 bn = e < 15 ? b[s][(e + 1) >> 2] : b[s ^ 1][0];
+                const v16f nx = __builtin_amdgcn_mfma_f32_16x16x1f32(an[(e + 1) & 3], bn[(e + 1) & 3], v16f{}, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[v] += pr[v];
+                pr = nx;
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);    /* one MFMA, */
+                __builtin_amdgcn_sched_group_barrier(0x2, 16, 0);   /* then the adds */
+            }
+        };
+        for (int g = 0; g < ng; g += 2) {
+            group(0, g + 1);
+            if (g + 1 >= ng) break;
+            group(1, g + 2);
         }
+    }
+    /* the rest: a product past its row's position is dropped, not added (0 * inf would not be 0) */
+    int P[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) P[k] = p0 + (r0 + 4 * (lane >> 4) + k) / R;
+    const int pmax = p0 + min(r0 + PF_VROWS - 1, nrows - 1) / R;
+    for (int u = 16 * ng; u <= pmax; u += 4) {
+        const f32x4 at = A4[u >> 2], vt = vtile(u >> 2);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const v16f pr = __builtin_amdgcn_mfma_f32_16x16x1f32(at[e], vt[e], v16f{}, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[v] = u + e <= P[v & 3] ? acc[v] + pr[v] : acc[v];
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        const int r = r0 + 4 * (lane >> 4) + (v & 3), ic = 64 * slab + 16 * (v >> 2) + (lane & 15);
+        if (r < nrows && ic < HD) att[((size_t)(r / R) * H + kvh * R + r % R) * HD + ic] = acc[v];
     }
 }
 
@@ -1187,29 +1218,25 @@ int launch_pf_attn(int hd, int H, int KV, int max_ctx, int p0, int ntok, float *
     const int has_qn = q_norm != nullptr, has_kn = k_norm != nullptr;
     if (!q_norm) q_norm = q;   /* read and dropped */
     if (!k_norm) k_norm = q;
-    const int R = H / KV, HB = R % 8 == 0 ? 8 : R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1;
-    const dim3 gsc((unsigned)((p0 + ntok + 63) / 64), (unsigned)((ntok + PF_TOK - 1) / PF_TOK), (unsigned)KV);
-    const dim3 gpv((unsigned)(KV * ((hd + 63) / 64)), (unsigned)((ntok + PF_TOK - 1) / PF_TOK));
-#define TLM_PF_HB(W, B)                                                                                         \
-    case B:                                                                                                     \
-        hipLaunchKernelGGL((k_pf_scores<W, B>), gsc, dim3(NT), 0, s, (const float *)q, (const float *)kc,      \
-                           scores, H, KV, max_ctx, p0, ntok, SL);                                               \
-        hipLaunchKernelGGL(k_pf_softmax, dim3((unsigned)H, (unsigned)ntok), dim3(NT), 0, s, scores, H, p0, SL); \
-        hipLaunchKernelGGL((k_pf_pv<W, B>), gpv, dim3(NT), 0, s, (const float *)scores, (const float *)vc, att, \
-                           H, KV, max_ctx, p0, ntok, SL);                                                       \
-        break;
+    const int rows = ntok * (H / KV);   /* of one key head */
+    const int rs = NT / 64 * PF_SROWS, rv = NT / 64 / pf_slabs(hd) * PF_VROWS;
+    const dim3 gsc((unsigned)((p0 + ntok + 63) / 64), (unsigned)((rows + rs - 1) / rs), (unsigned)KV);
+    const dim3 gpv((unsigned)KV, (unsigned)((rows + rv - 1) / rv));
 #define TLM_PF(W)                                                                                                \
     case W:                                                                                                      \
         hipLaunchKernelGGL((k_pf_prep<W>), dim3((unsigned)ntok), dim3(NT), 0, s, q, kx, vx, q_norm, k_norm,     \
                            has_qn, has_kn, cs, sn, kc, vc, H, KV, max_ctx, p0, eps);                            \
-        switch (HB) { TLM_PF_HB(W, 8) TLM_PF_HB(W, 4) TLM_PF_HB(W, 2) TLM_PF_HB(W, 1) }                          \
+        hipLaunchKernelGGL((k_pf_scores<W>), gsc, dim3(NT), 0, s, (const float *)q, (const float *)kc, scores,  \
+                           H, KV, max_ctx, p0, ntok, SL);                                                       \
+        hipLaunchKernelGGL(k_pf_softmax, dim3((unsigned)H, (unsigned)ntok), dim3(NT), 0, s, scores, H, p0, SL); \
+        hipLaunchKernelGGL((k_pf_pv<W>), gpv, dim3(NT), 0, s, (const float *)scores, (const float *)vc, att, H, \
+                           KV, max_ctx, p0, ntok, SL);                                                          \
         break;
     switch (hd) {
         TLM_PF(32) TLM_PF(64) TLM_PF(96) TLM_PF(128)
     default: return tlmh_seterr(TLM_HIP_EUNSUP, "model prefill: head width %d", hd);
     }
 #undef TLM_PF
-#undef TLM_PF_HB
     return tlmh_check(hipGetLastError(), "model: prefill attention");
 }
 
