@@ -147,6 +147,30 @@ def test_matvec_tiles_ranges(hip, dev, dt):
 
 
 @pytest.mark.parametrize("dt", INT)
+@pytest.mark.parametrize("nb,rows", [(1, 17), (4, 33), (5, 9), (8, 7), (9, 25), (16, 5), (17, 18), (33, 6), (64, 3),
+                                     (65, 6), (129, 5)])
+def test_matvec_rows_groups(hip, dev, dt, nb, rows):
+    """Rows per group (16 / 8 / 4 by the row's blocks), part groups, and rows
+    of one block more than a chunk (64 blocks; Q8_0 128), at an odd stride and
+    base, against the oracle bit for bit."""
+    rng = np.random.default_rng(100 * nb + dt)
+    n = nb * oracle.BLOCK[dt][0]
+    tight = oracle.row_bytes(dt, n)
+    rb, off = tight + 5, 7
+    mem = np.full(rb * rows + off, 0xA5, np.uint8)
+    for r in range(rows):
+        mem[off + rb * r: off + rb * r + tight] = make_wrow(rng, dt, n, r % 5)
+    act = make_act(rng, dt, n, 0)
+    want = oracle.matvec_rows(dt, mem, rb, act, n, 0, rows, offset=off)
+    y = torch.full((rows + 1,), -12345.0, device=dev)
+    hip.matvec_rows(dt, to_dev(mem, dev), rb, to_dev(act, dev), n, 0, rows, y=y, offset=off)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert got[rows] == -12345.0
+    assert np.all(same(got[:rows], want))
+
+
+@pytest.mark.parametrize("dt", INT)
 @pytest.mark.parametrize("rows,n", [(16, 256), (48, 512), (37, 768), (768, 2048), (2048, 768), (100, 4096),
                                     (64, 8192), (4096, 8192), (4100, 2048), (16400, 512), (16400, 2048),
                                     (16384, 4096)])

@@ -10,8 +10,8 @@
  *
  * Two layouts:
  *   plain  - the reference's row-major bytes, any stride / base offset
- *            (the drop-in tlm_matvec_rows path).  One lane per block,
- *            byte-granular weight reads.
+ *            (the drop-in tlm_matvec_rows path).  The packed path's lanes and
+ *            integer code on unaligned vector loads.
  *   packed - tile layout produced on device by launch_pack (see
  *            packed_bytes): rows grouped in tiles of 16; the tile's rows are
  *            contiguous per block column, and the f16 scale of Q6_K / Q8_0
@@ -30,102 +30,67 @@ namespace {
 /* ======================================================================
  * plain layout
  * ==================================================================== */
-__device__ __forceinline__ uint32_t ld_u8(const uint8_t *p) { return *p; }
 __device__ __forceinline__ uint32_t ld_u16u(const uint8_t *p) { return (uint32_t)p[0] | ((uint32_t)p[1] << 8); }
 
-/* Integer sums of one plain block (any alignment) against a 4-byte aligned
- * activation block - the per-element rules of src/lib/tlm_quant.c:778-902. */
-template <int DT>
-__device__ void plain_block(const uint8_t *w, const uint8_t *a, int32_t &is, int32_t &ms) {
-    is = 0;
-    ms = 0;
-    const int8_t *x = (const int8_t *)(a + 4);
-    if constexpr (DT == DT_Q8_0) {
-        for (int i = 0; i < 32; i++) is += (int32_t)(int8_t)w[2 + i] * x[i];
-    } else if constexpr (DT == DT_Q8_K) {
-        for (int i = 0; i < 256; i++) is += (int32_t)(int8_t)w[4 + i] * x[i];
-    } else if constexpr (DT == DT_Q6_K) {
-        const int16_t *bs = (const int16_t *)(a + 260);
-        for (int g = 0; g < 16; g++) {
-            int32_t gs = 0;
-            for (int k = 0; k < 16; k++) {
-                int e = 16 * g + k, h = e >> 7, q = (e >> 5) & 3, l = e & 31;
-                uint32_t nib = w[64 * h + 32 * (q & 1) + l];
-                nib = (q & 2) ? (nib >> 4) : (nib & 15u);
-                uint32_t hi = (w[128 + 32 * h + l] >> (2 * q)) & 3u;
-                gs += (int32_t)(nib | (hi << 4)) * x[e];
-            }
-            is += (int32_t)(int8_t)w[192 + g] * (gs - 32 * (int32_t)bs[g]);
-        }
-    } else {   /* Q4_K / Q5_K */
-        constexpr bool Q5 = DT == DT_Q5_K;
-        const uint8_t *qs = w + (Q5 ? 48 : 16), *s12 = w + 4;
-        const int16_t *bs = (const int16_t *)(a + 260);
-        for (int sb = 0; sb < 8; sb++) {
-            int c = sb >> 1, hb = sb & 1;
-            uint32_t sc, mn;
-            if (sb < 4) { sc = s12[sb] & 63u; mn = s12[4 + sb] & 63u; }
-            else {
-                sc = (s12[sb + 4] & 15u) | ((uint32_t)(s12[sb - 4] >> 6) << 4);
-                mn = ((uint32_t)s12[sb + 4] >> 4) | ((uint32_t)(s12[sb] >> 6) << 4);
-            }
-            int32_t s = 0;
-            for (int l = 0; l < 32; l++) {
-                uint32_t code = hb ? (qs[32 * c + l] >> 4) : (qs[32 * c + l] & 15u);
-                if (Q5) code |= ((w[16 + l] >> (2 * c + hb)) & 1u) << 4;
-                s += (int32_t)code * x[32 * sb + l];
-            }
-            is += (int32_t)sc * s;
-            ms += (int32_t)mn * ((int32_t)bs[2 * sb] + (int32_t)bs[2 * sb + 1]);
-        }
-    }
+/* A group takes rpg rows: the items (row, block) of a chunk of blocks go
+ * through run_items with the packed path's lanes per item and integer code
+ * (consecutive items are consecutive blocks of a row), the chunk's
+ * activation staged in LDS, then one thread per row runs its chain over the
+ * parked sums.  PLAIN_IPL items a lane bound a chunk: 64 blocks of 4 rows
+ * (Q8_0: 128), in 23 KB of LDS.  Bound: one round trip of each chunk's loads,
+ * and the launch.  4096 x 4096 Q6_K (14.1 MB) takes 6.8 us
+ * (2.1 TB/s); one lane per block with byte loads took 53 us, 48 of a wave's
+ * 64 lanes idle at 16 blocks a row.
+ * Rows per group: one round of one item a lane for the narrowest rows (a
+ * group of 4 rows of 4 blocks would use 16 of its 64 item slots), 4 from 16
+ * blocks (Q8_0: 32) on, where groups to fill the chip are what is short. */
+constexpr int PLAIN_IPL = 4;
+__host__ __device__ constexpr int plain_slots(int dt) { return GROUP_THREADS / (dt == DT_Q8_0 ? 2 : 4); }
+__host__ __device__ constexpr int plain_nbc(int dt) { return plain_slots(dt) * PLAIN_IPL / 4; }
+__host__ __device__ static inline int plain_rpg(int dt, int64_t nb) {
+    return nb * 16 <= plain_slots(dt) ? 16 : nb * 8 <= plain_slots(dt) ? 8 : 4;
+}
+static size_t plain_lds_bytes(int dt, int64_t nb) {
+    const int cap = nb < plain_nbc(dt) ? (int)nb : plain_nbc(dt);
+    return ((stage_bytes(dt_act_kind(dt), cap) + 15) & ~(size_t)15) + park_bytes(cap * plain_rpg(dt, nb));
 }
 
-template <int DT>
-__device__ __forceinline__ void plain_scales(const uint8_t *w, const uint8_t *a, float &dA, float &dM) {
-    float da = *(const float *)a;
-    if constexpr (DT == DT_Q6_K) { dA = f16_to_f32(ld_u16u(w + 208)) * da; dM = 0.0f; }
-    else if constexpr (DT == DT_Q8_0) { dA = f16_to_f32(ld_u16u(w)) * da; dM = 0.0f; }
-    else if constexpr (DT == DT_Q8_K) {
-        uint32_t u = ld_u16u(w) | (ld_u16u(w + 2) << 16);
-        dA = __uint_as_float(u) * da;
-        dM = 0.0f;
-    } else { dA = f16_to_f32(ld_u16u(w)) * da; dM = f16_to_f32(ld_u16u(w + 2)) * da; }
-}
-
-/* One wave per row, 4 rows per work-group.  Lanes take blocks lane, lane+64,
- * ...; the chain runs in every lane (same values) over shuffled block results
- * in ascending order. */
 template <int DT>
 __device__ __forceinline__ void mv_plain_rows(const uint8_t *__restrict__ W, size_t row_bytes,
                                               const uint8_t *__restrict__ act, float *__restrict__ y, int64_t n,
                                               int64_t r0, int64_t r1, int64_t bid) {
-    constexpr int BV = DT == DT_Q8_0 ? 32 : 256;
+    using F = Plain<DT>;
     constexpr int AB = DT == DT_Q8_0 ? 36 : 292;
     constexpr int WB = DT == DT_Q8_0 ? 34 : DT == DT_Q4_K ? 144 : DT == DT_Q5_K ? 176 : DT == DT_Q6_K ? 210 : 292;
     constexpr bool AFF = DT == DT_Q4_K || DT == DT_Q5_K;
-    const int lane = threadIdx.x & 63;
-    const int64_t row = r0 + bid * 4 + (threadIdx.x >> 6);
-    if (row >= r1) return;
-    const uint8_t *w = W + (size_t)row * row_bytes;
-    const int64_t nb = n / BV;
+    constexpr int NBC = plain_nbc(DT);
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int64_t nb = n / F::BV;
+    const int rpg = plain_rpg(DT, nb), kind = dt_act_kind(DT), cap = nb < NBC ? (int)nb : NBC;
+    const int64_t row0 = r0 + bid * rpg;
+    const int nr = r1 - row0 < rpg ? (int)(r1 - row0) : rpg;
+    const Park park = park_at(lds + ((stage_bytes(kind, cap) + 15) & ~(size_t)15), cap * rpg);
     float acc = 0.0f;
-    for (int64_t base = 0; base < nb; base += 64) {
-        int64_t b = base + lane;
-        int32_t is = 0, ms = 0;
-        float dA = 0.0f, dM = 0.0f;
-        if (b < nb) {
-            plain_block<DT>(w + (size_t)b * WB, act + (size_t)b * AB, is, ms);
-            plain_scales<DT>(w + (size_t)b * WB, act + (size_t)b * AB, dA, dM);
-        }
-        float fis = (float)is, fms = (float)ms;
-        int cnt = (int)(nb - base < 64 ? nb - base : 64);
-        for (int j = 0; j < cnt; j++) {
-            acc = fmaf(__shfl(dA, j, 64), __shfl(fis, j, 64), acc);
-            if (AFF) acc = fmaf(-__shfl(dM, j, 64), __shfl(fms, j, 64), acc);
-        }
+    for (int64_t b0 = 0; b0 < nb; b0 += NBC) {   /* uniform */
+        const int ncb = nb - b0 < NBC ? (int)(nb - b0) : NBC;
+        auto map = [&](int it, const uint8_t *&w, int64_t &un, int64_t &u, int &b, int &pk) {
+            const int i = it / ncb;
+            b = it - i * ncb;
+            w = W + (size_t)(row0 + i) * row_bytes + (size_t)(b0 + b) * WB;
+            un = u = 0;
+            pk = b * rpg + i;
+        };
+        auto stage = [&]() {
+            const XLds X = stage_act(kind, act + (size_t)b0 * AB, ncb, lds);
+            __syncthreads();
+            return X;
+        };
+        run_items<DT, PLAIN_IPL, false, F>(ncb * nr, map, stage, park);
+        __syncthreads();
+        if ((int)threadIdx.x < nr) acc = chain_park<AFF>(park, ncb, 0, rpg, threadIdx.x, acc);
+        __syncthreads();   /* the chunk is read */
     }
-    if (lane == 0) y[row] = acc;
+    if ((int)threadIdx.x < nr) y[row0 + threadIdx.x] = acc;
 }
 template <int DT>
 __global__ __launch_bounds__(256) void k_mv_plain_int(const uint8_t *__restrict__ W, size_t row_bytes,
@@ -662,7 +627,7 @@ __global__ __launch_bounds__(256) void k_mv_packed_seg(MvSegs sg, int nb, const 
  * src/lib/tlm_model.c:175-222): JOB_SEGS segments of any dtype, width,
  * layout and activation; segment s owns groups [first[s], first[s + 1]) and
  * every group runs its segment's body (a uniform switch): a 16-row tile of a
- * packed matrix, 4 plain rows of an integer format or 8 f32 rows. */
+ * packed matrix, plain_rpg plain rows of an integer format or 8 f32 rows. */
 enum { JK_PACKED = 0, JK_PACKED_MID = 1, JK_PLAIN = 2, JK_F32 = 3, JK_F32_UNALIGNED = 4 };
 struct JobSeg {
     const uint8_t *W, *act;
@@ -743,13 +708,16 @@ int launch_matvec_plain(int dt, const void *W, size_t row_bytes, const void *act
         else hipLaunchKernelGGL(k_mv_f32<false>, g, dim3(256), 0, s, w, row_bytes, (const float *)a, y, n, r0, r1);
         return tlmh_check(hipGetLastError(), "matvec f32 launch");
     }
-    dim3 g((unsigned)((rows + 3) / 4)), blk(256);
+    const int64_t nb = n / bv;
+    const int rpg = plain_rpg(dt, nb);
+    const size_t lds = plain_lds_bytes(dt, nb);
+    dim3 g((unsigned)((rows + rpg - 1) / rpg)), blk(256);
     switch (dt) {
-    case DT_Q8_0: hipLaunchKernelGGL(k_mv_plain_int<DT_Q8_0>, g, blk, 0, s, w, row_bytes, a, y, n, r0, r1); break;
-    case DT_Q4_K: hipLaunchKernelGGL(k_mv_plain_int<DT_Q4_K>, g, blk, 0, s, w, row_bytes, a, y, n, r0, r1); break;
-    case DT_Q5_K: hipLaunchKernelGGL(k_mv_plain_int<DT_Q5_K>, g, blk, 0, s, w, row_bytes, a, y, n, r0, r1); break;
-    case DT_Q6_K: hipLaunchKernelGGL(k_mv_plain_int<DT_Q6_K>, g, blk, 0, s, w, row_bytes, a, y, n, r0, r1); break;
-    case DT_Q8_K: hipLaunchKernelGGL(k_mv_plain_int<DT_Q8_K>, g, blk, 0, s, w, row_bytes, a, y, n, r0, r1); break;
+    case DT_Q8_0: hipLaunchKernelGGL(k_mv_plain_int<DT_Q8_0>, g, blk, lds, s, w, row_bytes, a, y, n, r0, r1); break;
+    case DT_Q4_K: hipLaunchKernelGGL(k_mv_plain_int<DT_Q4_K>, g, blk, lds, s, w, row_bytes, a, y, n, r0, r1); break;
+    case DT_Q5_K: hipLaunchKernelGGL(k_mv_plain_int<DT_Q5_K>, g, blk, lds, s, w, row_bytes, a, y, n, r0, r1); break;
+    case DT_Q6_K: hipLaunchKernelGGL(k_mv_plain_int<DT_Q6_K>, g, blk, lds, s, w, row_bytes, a, y, n, r0, r1); break;
+    case DT_Q8_K: hipLaunchKernelGGL(k_mv_plain_int<DT_Q8_K>, g, blk, lds, s, w, row_bytes, a, y, n, r0, r1); break;
     }
     return tlmh_check(hipGetLastError(), "matvec launch");
 }
@@ -919,8 +887,10 @@ int launch_mv_job(const tlm_hip_seg *segs, int nseg, hipStream_t s) {
                 kind = ((uintptr_t)g->W % 4 == 0 && g->row_bytes % 4 == 0) ? JK_F32 : JK_F32_UNALIGNED;
                 ng = (g->rows + 7) / 8;
             } else {
+                const int rpg = plain_rpg(g->dt, g->n / bv);
                 kind = JK_PLAIN;
-                ng = (g->rows + 3) / 4;
+                need = plain_lds_bytes(g->dt, g->n / bv);
+                ng = (g->rows + rpg - 1) / rpg;
             }
         }
         if (kind < 0) {

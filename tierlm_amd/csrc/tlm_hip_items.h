@@ -254,6 +254,53 @@ template <> struct Packed<DT_Q8_K> {
     }
 };
 
+/* ---- blocks of the reference's row layout -----------------------------------
+ * Plain<DT>: the packed item's lanes, registers and compute, loading a whole
+ * block at any byte address (W is the block; units and u are not used).  The
+ * unaligned vector types make every load a single instruction all the same
+ * (gfx950 takes unaligned vector loads). */
+typedef u32x4 u32x4_u __attribute__((aligned(1)));
+typedef u32x2 u32x2_u __attribute__((aligned(1)));
+typedef uint32_t u32_u __attribute__((aligned(1)));
+typedef uint16_t u16_u __attribute__((aligned(1)));
+template <int DT> struct Plain : Packed<DT> {
+    using Raw = typename Packed<DT>::Raw;
+    __device__ static __forceinline__ Raw load(const uint8_t *__restrict__ W, int64_t, int64_t, int q) {
+        const GAS uint8_t *blk = (const GAS uint8_t *)W;
+        Raw r;
+        if constexpr (DT == DT_Q6_K) {
+            const int h = q >> 1, p = q & 1;
+            r.A = *(const GAS u32x4_u *)(blk + 64 * h + 16 * p);
+            r.B = *(const GAS u32x4_u *)(blk + 64 * h + 32 + 16 * p);
+            r.C = *(const GAS u32x4_u *)(blk + 128 + 32 * h + 16 * p);
+            r.S = *(const GAS u32x2_u *)(blk + 192 + 8 * h);
+            r.dw = *(const GAS u16_u *)(blk + 208);
+        } else if constexpr (DT == DT_Q8_0) {
+            r.W = *(const GAS u32x4_u *)(blk + 2 + 16 * q);
+            r.dw = *(const GAS u16_u *)blk;
+        } else if constexpr (DT == DT_Q8_K) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const u32x4 v = *(const GAS u32x4_u *)(blk + 4 + 64 * q + 16 * j);
+#pragma unroll
+                for (int k = 0; k < 4; k++) r.w[4 * j + k] = v[k];
+            }
+            r.d = *(const GAS u32_u *)blk;
+        } else {
+            constexpr int QS = Packed<DT>::QS;
+            r.H = *(const GAS u32x4_u *)blk;
+            r.Q0 = *(const GAS u32x4_u *)(blk + QS + 32 * q);
+            r.Q1 = *(const GAS u32x4_u *)(blk + QS + 32 * q + 16);
+            r.P0 = r.P1 = u32x4{0, 0, 0, 0};
+            if constexpr (DT == DT_Q5_K) {
+                r.P0 = *(const GAS u32x4_u *)(blk + 16);
+                r.P1 = *(const GAS u32x4_u *)(blk + 32);
+            }
+        }
+        return r;
+    }
+};
+
 /* ---- parked item results in LDS: [item] for one matrix tile ---------------- */
 struct Park {
     LAS int32_t *is, *ms;
@@ -278,9 +325,8 @@ __device__ __forceinline__ static Park park_at(uint8_t *p, int nitems) {
  * load the last item's bytes and are dropped: with many items per lane the
  * compiler keeps branch-free loads in flight together, where a branch per
  * item made it wait between them.  Returns the XLds that stage() produced. */
-template <int DT, int IPL, bool CLAMP = false, class Map, class Stage>
+template <int DT, int IPL, bool CLAMP = false, class F = Packed<DT>, class Map, class Stage>
 __device__ __forceinline__ XLds run_items(int nitems, Map map, Stage stage, Park park) {
-    using F = Packed<DT>;
     constexpr bool AFF = DT == DT_Q4_K || DT == DT_Q5_K;
     const int slots = GROUP_THREADS / F::LPI;
     const int q = threadIdx.x % F::LPI, slot = threadIdx.x / F::LPI;
