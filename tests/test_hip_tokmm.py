@@ -87,3 +87,34 @@ def test_tokmm_rejects_bad_arguments(hip, dev):
         hip.matmul_tokens(oracle.Q6_K, Wp, 16, 100, act, 2)      # n not a multiple of 256
     with pytest.raises(HipError):
         hip.matmul_tokens(oracle.Q8_K, Wp, 16, 256, act, 2)      # dtype without a token kernel
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_tokmm_q8_0_scale_range(hip, dev, mode):
+    """Q8_0 scale products from the matrix cores: weight scales over every
+    binary16 class (subnormal, largest, signed zero, infinity, NaN) and
+    activation scales down to where the product is subnormal, part tiles of
+    rows and tokens, against the decode matvec bit for bit."""
+    rows, n, ntok = 45, 512, 37
+    rng = np.random.default_rng(5 + mode)
+    W = oracle.quantize_row(oracle.Q8_0, rng.standard_normal((rows, n)).astype(np.float32) * 0.02).reshape(rows, -1)
+    d = W.reshape(rows, n // 32, 34)
+    if mode:   # the special values of binary16
+        sc = rng.choice(np.array([0x0001, 0x8001, 0x03FF, 0x0400, 0x7BFF, 0xFBFF, 0x0000, 0x8000, 0x7C00, 0x7E01],
+                                 np.uint16), size=(rows, n // 32))
+    else:
+        sc = rng.integers(0, 0x7C00, size=(rows, n // 32)).astype(np.uint16) | \
+            (rng.integers(0, 2, size=(rows, n // 32)).astype(np.uint16) << 15)
+    d[:, :, 0:2] = np.ascontiguousarray(sc).view(np.uint8).reshape(rows, n // 32, 2)
+    x = rng.standard_normal((ntok, n)).astype(np.float32)
+    x *= np.exp2(rng.integers(-125, 40, size=(ntok, n // 32)).repeat(32, 1)).astype(np.float32)
+    Wd = torch.from_numpy(W.reshape(-1).copy()).to(dev)
+    P = hip.pack(oracle.Q8_0, Wd, W.shape[1], rows, n)
+    acts = [oracle.quantize_act(oracle.Q8_0, x[t]) for t in range(ntok)]
+    got = hip.matmul_tokens(oracle.Q8_0, P, rows, n, torch.from_numpy(np.concatenate(acts)).to(dev), ntok)
+    torch.cuda.synchronize()
+    got = got.cpu().numpy().reshape(ntok, rows)
+    for t in range(ntok):
+        want = hip.matvec_packed(oracle.Q8_0, P, rows, n, torch.from_numpy(acts[t]).to(dev)).cpu().numpy()
+        same = (got[t].view(np.uint32) == want.view(np.uint32)) | (np.isnan(got[t]) & np.isnan(want))
+        assert same.all(), (t, got[t][~same], want[~same])

@@ -44,6 +44,7 @@ constexpr int TM_WAVES = 4;      /* waves per group */
 
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v32f __attribute__((ext_vector_type(32)));
 
 __host__ __device__ constexpr bool tile_dt(int dt) {
     return dt == DT_Q4_K || dt == DT_Q5_K || dt == DT_Q6_K || dt == DT_Q8_0;
@@ -91,9 +92,9 @@ template <> struct WRaw<DT_Q5_K> {   /* d | dmin, scales[12]; qs bytes 32c + 16 
 template <> struct WRaw<DT_Q4_K> {
     u32x4 hdr, qs[4];
 };
-template <> struct WRaw<DT_Q8_0> {   /* eight blocks: this lane's 16 code bytes of each, and each block's d */
+template <> struct WRaw<DT_Q8_0> {   /* eight blocks: this lane's 16 code bytes of each; d of blocks 2k + half */
     u32x4 q[8];
-    uint32_t d[8];
+    uint32_t d[4];
 };
 
 /* block 0 of a chain's row: its unit, and (Q6_K) its d in the d plane */
@@ -128,10 +129,10 @@ __device__ __forceinline__ WRaw<DT> wload(const Chain &ch, int b, int half) {
         r.d = ch.dp[b * TILE_ROWS];
     } else if constexpr (DT == DT_Q8_0) {   /* b counts staged 256-value groups: blocks 8b .. 8b + 7 */
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int i = 0; i < 8; i++)
             r.q[i] = *(const GAS u32x4 *)(ch.unit + (size_t)(8 * b + i) * (TILE_ROWS * 32) + 16 * half);
-            r.d[i] = ch.dp[(8 * b + i) * TILE_ROWS];
-        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) r.d[k] = ch.dp[(8 * b + 2 * k + half) * TILE_ROWS];
     } else {
         constexpr int QS = DT == DT_Q5_K ? 48 : 16;
         r.hdr = *(const GAS u32x4 *)u;
@@ -224,6 +225,13 @@ __device__ __forceinline__ void stage_store(LAS uint8_t *buf, const StageRegs &r
     }
 }
 
+/* f16_to_f32 as v_cvt_f32_f16: the same value for every input (subnormals
+ * kept, a NaN quieted with its payload); no load is held up here by a
+ * conversion the compiler could branch around */
+__device__ __forceinline__ float f16_cvt(uint32_t h) {
+    return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
+}
+
 __device__ __forceinline__ long pack2(uint32_t lo, uint32_t hi) {
     return (long)(((unsigned long long)hi << 32) | lo);
 }
@@ -269,7 +277,7 @@ __device__ __forceinline__ void block_chain(const WRaw<DT_Q6_K> &w, const LAS ui
     const v4i scv = {(int)w.sc.x, (int)w.sc.y, (int)w.sc.z, (int)w.sc.w};
     const v16i m = group_sum_term(sa, scv, half);       /* sum_g sc_g S_g, |.| <= 2^22 */
     const LAS float *dd = (const LAS float *)(buf + S::D) + 4 * half;
-    const float dwf = f16_to_f32(w.d);
+    const float dwf = f16_cvt(w.d);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const f32x4 da = *(const LAS f32x4 *)(dd + 8 * q);
@@ -283,39 +291,46 @@ __device__ __forceinline__ void block_chain(const WRaw<DT_Q6_K> &w, const LAS ui
 }
 
 /* eight Q8_0 blocks: per block the exact int32 sum, then the row's fma
- * (d_w d_a, isum) in ascending block order, as the decode dot */
+ * (d_w d_a, isum) in ascending block order, as the decode dot.  The rounded
+ * products d_w d_a of a pair of blocks over the tile are an outer product: one
+ * v_mfma_f32_32x32x1 (two blocks of K = 1, C = 0: v_mul_f32's rounding,
+ * subnormals included) in the layout of the integer sums.  That leaves the
+ * VALU a conversion and an fma per output and block, and the token scales one
+ * LDS word per lane and pair; multiplied on the VALU they were four 16-byte
+ * broadcasts per block, which LDS could not keep up with.  4096 x 2048, 1024
+ * tokens (8.6 G products): 54 -> 41 us.  Bound: VALU issue, with two waves a
+ * SIMD (208 registers) to cover the MFMAs and barriers. */
 __device__ __forceinline__ void block_chain(const WRaw<DT_Q8_0> &w, const LAS uint8_t *buf, int t, int half,
                                             float (&acc)[16]) {
     using S = Stage<DT_Q8_0>;
     const LAS uint8_t *cod = buf + t * S::CS + 16 * half;
+    const LAS float *dd = (const LAS float *)(buf + S::D) + 32 * half + t;
+    /* the empty statements keep their order with the ones behind the chains:
+     * two integer products and two pairs' scales are live - hoisting all of
+     * them spills */
     auto mm = [&](int i) {
         v4i ax = *(const LAS v4i *)(cod + 32 * i);
-        /* ordered after the previous block's chain (the volatile statements
-         * below keep their order): at most two products live - hoisting all
-         * eight 16-register results spills */
         asm volatile("" : "+v"(ax));
         const v4i bw = {(int)w.q[i].x, (int)w.q[i].y, (int)w.q[i].z, (int)w.q[i].w};
         return __builtin_amdgcn_mfma_i32_32x32x32_i8(ax, bw, v16i{}, 0, 0, 0);
     };
-    /* block i + 1's product is issued before block i's chain */
+    auto scales = [&](int k) {   /* blocks 2k (elements 0..15) and 2k + 1 (16..31) */
+        float da = dd[64 * k];
+        asm volatile("" : "+v"(da));
+        return __builtin_amdgcn_mfma_f32_32x32x1f32(da, f16_cvt(w.d[k]), v32f{}, 0, 0, 0);
+    };
+    v32f sc = scales(0), scn = sc;
     v16i pn = mm(0);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
+    for (int i = 0; i < 8; i++) {   /* block i + 1's product is issued before block i's chain */
         const v16i p = pn;
         if (i < 7) pn = mm(i + 1);
-        const LAS float *dd = (const LAS float *)(buf + S::D) + 32 * i + 4 * half;
-        const float dw = f16_to_f32(w.d[i]);
+        if ((i & 1) && i < 7) scn = scales((i + 1) / 2);
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const f32x4 da = *(const LAS f32x4 *)(dd + 8 * q);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int v = 4 * q + k;
-                acc[v] = fmaf(dw * da[k], (float)p[v], acc[v]);
-            }
-        }
+        for (int v = 0; v < 16; v++) acc[v] = fmaf(sc[16 * (i & 1) + v], (float)p[v], acc[v]);
 #pragma unroll
         for (int v = 0; v < 16; v++) asm volatile("" : "+v"(acc[v]));
+        if (i & 1) sc = scn;
     }
 }
 
@@ -354,7 +369,7 @@ __device__ __forceinline__ void block_chain(const WRaw<DT> &w, const LAS uint8_t
     const v4i mnv = {(int)mn0, (int)mn1, 0, 0};
     const v16i ms = group_sum_term(sa, mnv, half);      /* msum */
     const LAS float *dd = (const LAS float *)(buf + S::D) + 4 * half;
-    const float dw = f16_to_f32(w.hdr.x & 0xFFFFu), dmw = f16_to_f32(w.hdr.x >> 16);
+    const float dw = f16_cvt(w.hdr.x & 0xFFFFu), dmw = f16_cvt(w.hdr.x >> 16);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const f32x4 da = *(const LAS f32x4 *)(dd + 8 * q);
