@@ -147,3 +147,13 @@ def test_prefill_rejects_unsupported(hip, dev):
                           weights="random_codes")
     with pytest.raises(HipError):
         case.block.prefill(torch.zeros((4, 256), device=dev))
+
+
+@pytest.mark.parametrize("E,k,T,D,de", [(4, 2, 59, 512, 256), (4, 2, 60, 512, 256), (2, 2, 33, 256, 512),
+                                        (2, 2, 64, 512, 256), (3, 2, 97, 768, 256), (2, 1, 131, 256, 256)])
+def test_prefill_wide_tiles(hip, dev, E, k, T, D, de):
+    """Q6_K experts around the mean of slots per expert where tiles take 64
+    slots (59 tokens: below, 60: at it), tiles of 33, 64 and one slot, an odd
+    number of blocks, against the decode block per token."""
+    case = build_moe_case(D=D, de=de, E=E, k=k, expert_dt=oracle.Q6_K, seed=T, device=dev)
+    prefill_vs_decode(case, dev, T, seed=T + 1)

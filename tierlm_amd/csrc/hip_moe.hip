@@ -950,8 +950,19 @@ struct PfLayout {
     size_t sact, sg, su, sh, sout, sgate, sact_stride;   /* sact_stride: the larger token row */
     size_t tstride, hq_stride, total;
     int64_t T;
-    int MT;
+    int MT, tt;        /* tiles of the table; slots per tile */
 };
+
+/* Slots per tile: 64 for Q6_K once the experts average PF_WIDE_MEAN slots
+ * (the wide tile: one pass over an expert's weights for up to 64 tokens, its
+ * scales applied once), else 32: below that most experts fit one 32-slot tile,
+ * which leaves three waves a SIMD instead of two.  128 experts of 768 x 2048,
+ * top 8, gate/up + down: 512 tokens (mean 32) 192 -> 174 us, a prompt's chunks
+ * of 682 (mean 43) 191 -> 154 us. */
+constexpr int PF_WIDE_MEAN = 30;
+inline int pf_tile_slots(const tlm_hip_moe_desc &d, int64_t T) {
+    return d.expert_dt == DT_Q6_K && T * d.k >= (int64_t)PF_WIDE_MEAN * d.E ? tokmm::Wide::TOK : tokmm::TM_TOK;
+}
 
 inline PfLayout pf_layout(const tlm_hip_moe_desc &d, int64_t T) {
     PfLayout P;
@@ -959,7 +970,8 @@ inline PfLayout pf_layout(const tlm_hip_moe_desc &d, int64_t T) {
     const size_t pairs = (size_t)T * d.k;
     size_t o = 0;
     P.T = T;
-    P.MT = (int)(pairs / tokmm::TM_TOK + d.E);
+    P.tt = pf_tile_slots(d, T);
+    P.MT = (int)(pairs / P.tt + d.E);
     P.tstride = L.total;
     P.hq_stride = al256(stage_bytes(DT_Q8_K, (int)(d.de / 256)));
     P.tok = o;      o += P.tstride * T;
@@ -968,7 +980,7 @@ inline PfLayout pf_layout(const tlm_hip_moe_desc &d, int64_t T) {
     P.pair_pos = o; o += al256(pairs * 4);
     P.slot_of = o;  o += al256(pairs * 4);
     P.slot_tok = o; o += al256(pairs * 4);
-    P.tiles = o;    o += al256((size_t)P.MT * 12);
+    P.tiles = o;    o += al256((pairs / tokmm::TM_TOK + d.E) * 12);
     P.hbuf = o;     o += al256(pairs * d.de * 4);
     P.hq = o;       o += P.hq_stride * pairs;
     P.out = o;      o += al256(pairs * d.D * 4);
@@ -1222,10 +1234,10 @@ __global__ __launch_bounds__(64) void k_publish_slot(int32_t *entry, int32_t v) 
 }
 
 /* One group: slots grouped by expert (order within an expert is free - every
- * slot is computed on its own), and the tile table of 32-slot runs. */
+ * slot is computed on its own), and the tile table of P.tt-slot runs. */
 __global__ __launch_bounds__(256) void k_pf_bucket(tlm_hip_moe_desc d, PfLayout P, uint8_t *ws) {
     __shared__ int s_cnt[MAXE], s_off[MAXE], s_toff[MAXE], s_wc[4], s_wt[4];
-    args_now(d.E, d.k, P.T, P.MT, P.pair_e, P.pair_pos, P.slot_of, P.slot_tok, P.tiles, ws);
+    args_now(d.E, d.k, P.T, P.MT, P.tt, P.pair_e, P.pair_pos, P.slot_of, P.slot_tok, P.tiles, ws);
     const int tid = threadIdx.x, E = d.E;
     const int npair = (int)(P.T * d.k);
     const GAS int32_t *pe = (const GAS int32_t *)(ws + P.pair_e);
@@ -1252,7 +1264,7 @@ __global__ __launch_bounds__(256) void k_pf_bucket(tlm_hip_moe_desc d, PfLayout 
     /* exclusive scans of slot counts and tile counts over the experts: wave
      * scans, then the wave totals */
     const int c = tid < E ? s_cnt[tid] : 0;
-    const int nt = (c + tokmm::TM_TOK - 1) / tokmm::TM_TOK;
+    const int nt = (c + P.tt - 1) / P.tt;
     const int lane = tid & 63, wave = tid >> 6;
     int ic = c, it = nt;
 #pragma unroll
@@ -1296,20 +1308,31 @@ __global__ __launch_bounds__(256) void k_pf_bucket(tlm_hip_moe_desc d, PfLayout 
         for (int q = 0; q < nt; q++) {
             const int ti = s_toff[tid] + q;
             tiles[3 * ti] = tid;
-            tiles[3 * ti + 1] = s_off[tid] + tokmm::TM_TOK * q;
-            tiles[3 * ti + 2] = c - tokmm::TM_TOK * q < tokmm::TM_TOK ? c - tokmm::TM_TOK * q : tokmm::TM_TOK;
+            tiles[3 * ti + 1] = s_off[tid] + P.tt * q;
+            tiles[3 * ti + 2] = c - P.tt * q < P.tt ? c - P.tt * q : P.tt;
         }
     }
     for (int ti = tiles_used + tid; ti < P.MT; ti += 256) tiles[3 * ti] = -1;
 }
 
-/* Rows of gate and up: 64 rows per group over the tile's (up to 32) slots of
+/* Rows of gate and up: 64 rows per group over the tile's (up to TT) slots of
  * one expert - waves 0-1 stream gate rows, waves 2-3 the same rows of up -
- * then, through LDS, h = silu(g) * u per (slot, row) by all four waves. */
-template <int DT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_pf_gateup(tlm_hip_moe_desc d, WsLayout L, PfLayout P, uint8_t *ws) {
-    __shared__ __align__(16) uint8_t s_tile[tokmm::tile_lds_bytes<DT>()];
-    static_assert(tokmm::tile_lds_bytes<DT>() >= 2 * 32 * 64 * 4, "g / u area");
+ * then, through LDS, h = silu(g) * u per (slot, row) by all four waves.  TT is
+ * 32, or 64 (the wide tile, Q6_K). */
+template <int DT, int TT> constexpr int pf_lds_bytes() {
+    return TT == tokmm::TM_TOK ? tokmm::tile_lds_bytes<DT>() : tokmm::wide_lds_bytes();
+}
+template <int DT, int TT>
+__device__ __forceinline__ void pf_tile_run(const tokmm::Chain &ch, int nb, const GAS uint8_t *x,
+                                            LAS uint8_t *lds, float (&acc)[TT / 2]) {
+    if constexpr (TT == tokmm::TM_TOK) tokmm::tile_run<DT, true>(ch, nb, x, lds, acc);
+    else tokmm::tile_run_wide(ch, nb, x, lds, acc);
+}
+template <int DT, int TT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TT == 32 ? 3 : 2))) void k_pf_gateup(tlm_hip_moe_desc d, WsLayout L, PfLayout P, uint8_t *ws) {
+    static_assert(TT == tokmm::TM_TOK || (TT == tokmm::Wide::TOK && DT == DT_Q6_K), "tiles");
+    __shared__ __align__(16) uint8_t s_tile[pf_lds_bytes<DT, TT>()];
+    static_assert(pf_lds_bytes<DT, TT>() >= 2 * TT * 64 * 4, "g / u area");
     args_now(d.D, d.de, d.experts, L.xe, P.tok, P.tstride, P.tiles, P.slot_tok, P.hbuf, ws);
     const GAS int32_t *tl = (const GAS int32_t *)(ws + P.tiles) + 3 * blockIdx.y;
     const int e = tl[0];
@@ -1321,32 +1344,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     const int nb = (int)(d.D / 256);
     const int64_t units = (rows / TILE_ROWS) * nb * TILE_ROWS;
     const int64_t ubase = (rr / TILE_ROWS) * nb * TILE_ROWS + rr % TILE_ROWS;
-    const int js = (int)threadIdx.x >> 3;                  /* the token this thread stages */
+    const int js = (int)threadIdx.x * TT / GROUP_THREADS;  /* the token this thread stages */
     const int slot = s0 + (js < n ? js : n - 1);
     const int tok = ((const GAS int32_t *)(ws + P.slot_tok))[slot];
     const GAS uint8_t *x = (const GAS uint8_t *)(ws + P.tok + (size_t)tok * P.tstride + L.xe);
     const GAS uint64_t *xt = (const GAS uint64_t *)d.experts;
     if (!xt[3 * e]) return;   /* an expert outside this pass (its matrices in no slot): uniform over the group */
     const tokmm::Chain ch = tokmm::chain_at<DT>((const uint8_t *)xt[3 * e + up], units, ubase);
-    float acc[16];
-    tokmm::tile_run<DT, true>(ch, nb, x, (LAS uint8_t *)s_tile, acc);
+    float acc[TT / 2];
+    pf_tile_run<DT, TT>(ch, nb, x, (LAS uint8_t *)s_tile, acc);
     /* the tile ended on a barrier: its LDS takes g and u of the group's 64
-     * rows x 32 slots ([gate|up][slot][row]), then every thread forms 8 of
-     * the h values (slots past the tile's last are skipped) */
+     * rows x TT slots ([gate|up][slot][row]), then every thread forms TT / 4
+     * of the h values (slots past the tile's last are skipped) */
     LAS float *gu = (LAS float *)s_tile;
     const int rl = (wave & 1) * 32 + (lane & 31);
 #pragma unroll
-    for (int v = 0; v < 16; v++) gu[(up * 32 + 8 * (v >> 2) + 4 * half + (v & 3)) * 64 + rl] = acc[v];
+    for (int v = 0; v < TT / 2; v++) gu[(up * TT + 8 * (v >> 2) + 4 * half + (v & 3)) * 64 + rl] = acc[v];
     __syncthreads();
     const int r2 = threadIdx.x & 63;
     const int64_t orow = (int64_t)blockIdx.x * 64 + r2;
     if (orow < rows) {
         GAS float *hb = (GAS float *)(ws + P.hbuf);
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
+        for (int q = 0; q < TT / 4; q++) {
             const int i = 4 * q + (threadIdx.x >> 6);
             if (i < n) {
-                const float g = gu[i * 64 + r2], u = gu[(32 + i) * 64 + r2];
+                const float g = gu[i * 64 + r2], u = gu[(TT + i) * 64 + r2];
                 hb[(size_t)(s0 + i) * rows + orow] = g / (1.0f + expf_ref(-g)) * u;
             }
         }
@@ -1367,9 +1390,9 @@ __global__ __launch_bounds__(64) void k_pf_hquant(tlm_hip_moe_desc d, PfLayout P
 
 /* Rows of down: 4 waves x 32 rows per group over the tile's slots of one
  * expert. */
-template <int DT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_pf_down(tlm_hip_moe_desc d, PfLayout P, uint8_t *ws) {
-    __shared__ __align__(16) uint8_t s_tile[tokmm::tile_lds_bytes<DT>()];
+template <int DT, int TT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TT == 32 ? 3 : 2))) void k_pf_down(tlm_hip_moe_desc d, PfLayout P, uint8_t *ws) {
+    __shared__ __align__(16) uint8_t s_tile[pf_lds_bytes<DT, TT>()];
     args_now(d.D, d.de, d.experts, P.tiles, P.hq, P.hq_stride, P.out, ws);
     const GAS int32_t *tl = (const GAS int32_t *)(ws + P.tiles) + 3 * blockIdx.y;
     const int e = tl[0];
@@ -1380,18 +1403,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     const int64_t rr = row < rows ? row : rows - 1;
     const int nb = (int)(d.de / 256);
     const int64_t units = (rows / TILE_ROWS) * nb * TILE_ROWS;
-    const int js = (int)threadIdx.x >> 3;
+    const int js = (int)threadIdx.x * TT / GROUP_THREADS;
     const int slot = s0 + (js < n ? js : n - 1);
     const GAS uint8_t *x = (const GAS uint8_t *)(ws + P.hq + (size_t)slot * P.hq_stride);
     const uint8_t *wd = (const uint8_t *)((const GAS uint64_t *)d.experts)[3 * e + 2];
     if (!wd) return;   /* an expert outside this pass: uniform over the group */
     const tokmm::Chain ch = tokmm::chain_at<DT>(wd, units, (rr / TILE_ROWS) * nb * TILE_ROWS + rr % TILE_ROWS);
-    float acc[16];
-    tokmm::tile_run<DT, true>(ch, nb, x, (LAS uint8_t *)s_tile, acc);
+    float acc[TT / 2];
+    pf_tile_run<DT, TT>(ch, nb, x, (LAS uint8_t *)s_tile, acc);
     if (row < rows) {
         GAS float *out = (GAS float *)(ws + P.out);
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
+        for (int v = 0; v < TT / 2; v++) {
             const int i = 8 * (v >> 2) + 4 * half + (v & 3);
             if (i < n) out[(size_t)(s0 + i) * rows + row] = acc[v];
         }
@@ -1737,15 +1760,21 @@ int launch_moe_prefill_experts(const tlm_hip_moe_desc *d, int64_t T, void *ws, h
     uint8_t *w8 = (uint8_t *)ws;
     const dim3 ggu((unsigned)((d->de + 63) / 64), (unsigned)P.MT), gdn((unsigned)((d->D + 127) / 128), (unsigned)P.MT);
     switch (d->expert_dt) {
-    case DT_Q4_K: hipLaunchKernelGGL(k_pf_gateup<DT_Q4_K>, ggu, dim3(256), 0, s, dv, L, P, w8); break;
-    case DT_Q5_K: hipLaunchKernelGGL(k_pf_gateup<DT_Q5_K>, ggu, dim3(256), 0, s, dv, L, P, w8); break;
-    default: hipLaunchKernelGGL(k_pf_gateup<DT_Q6_K>, ggu, dim3(256), 0, s, dv, L, P, w8); break;
+    case DT_Q4_K: hipLaunchKernelGGL((k_pf_gateup<DT_Q4_K, 32>), ggu, dim3(256), 0, s, dv, L, P, w8); break;
+    case DT_Q5_K: hipLaunchKernelGGL((k_pf_gateup<DT_Q5_K, 32>), ggu, dim3(256), 0, s, dv, L, P, w8); break;
+    default:
+        if (P.tt == 64) hipLaunchKernelGGL((k_pf_gateup<DT_Q6_K, 64>), ggu, dim3(256), 0, s, dv, L, P, w8);
+        else hipLaunchKernelGGL((k_pf_gateup<DT_Q6_K, 32>), ggu, dim3(256), 0, s, dv, L, P, w8);
+        break;
     }
     hipLaunchKernelGGL(k_pf_hquant, dim3((unsigned)(T * d->k), (unsigned)(d->de / 256)), dim3(64), 0, s, dv, P, w8);
     switch (d->expert_dt) {
-    case DT_Q4_K: hipLaunchKernelGGL(k_pf_down<DT_Q4_K>, gdn, dim3(256), 0, s, dv, P, w8); break;
-    case DT_Q5_K: hipLaunchKernelGGL(k_pf_down<DT_Q5_K>, gdn, dim3(256), 0, s, dv, P, w8); break;
-    default: hipLaunchKernelGGL(k_pf_down<DT_Q6_K>, gdn, dim3(256), 0, s, dv, P, w8); break;
+    case DT_Q4_K: hipLaunchKernelGGL((k_pf_down<DT_Q4_K, 32>), gdn, dim3(256), 0, s, dv, P, w8); break;
+    case DT_Q5_K: hipLaunchKernelGGL((k_pf_down<DT_Q5_K, 32>), gdn, dim3(256), 0, s, dv, P, w8); break;
+    default:
+        if (P.tt == 64) hipLaunchKernelGGL((k_pf_down<DT_Q6_K, 64>), gdn, dim3(256), 0, s, dv, P, w8);
+        else hipLaunchKernelGGL((k_pf_down<DT_Q6_K, 32>), gdn, dim3(256), 0, s, dv, P, w8);
+        break;
     }
     return tlmh_check(hipGetLastError(), "moe_prefill launch");
 }

@@ -426,6 +426,136 @@ __device__ __forceinline__ void tile_run(const Chain &ch, int nb, const GAS uint
     }
 }
 
+/* ---- Q6_K against up to 64 tokens -----------------------------------------
+ * The 32-token tile applies a group's scale to the 16 sums of each MFMA, one
+ * VALU multiply-add per 16 products: that, not the matrix pipe or HBM, bounds
+ * it.  Here the scale goes into the weights instead, once for all of the
+ * tile's tokens: w = sc (u - 32) (|w| <= 4096) is split into two int8 planes,
+ * w = 256 hi + lo with hi = (w + 128) >> 8, both planes accumulate over the
+ * whole block in the MFMA's own accumulators, and isum = 256 H + L once per
+ * block - the same integer as sum_g sc_g (sum u x - 32 S_g) for a block whose
+ * bsums are the sums of its codes, as every block this library quantises.
+ * The split costs 12 VALU instructions per four weights against 5 for the
+ * plain codes: about 600 instructions a block and lane for the 64 tokens
+ * against 500 for each 32 (215 registers, two waves a SIMD, against 168 and
+ * three). */
+struct Wide {
+    static constexpr int TOK = 64;
+    static constexpr int CS = 272;             /* 16-byte reads: lanes on distinct banks */
+    static constexpr int D = TOK * CS;         /* f32 d per token */
+    static constexpr int BYTES = D + TOK * 4;
+};
+constexpr int wide_lds_bytes() { return 2 * Wide::BYTES; }
+
+struct WRawWide {   /* ql pieces [h][qq & 1], qh [h]: the lane's 16 of each 32; scales; d */
+    u32x4 ql[4], qh[2], sc;
+    uint32_t d;
+};
+__device__ __forceinline__ WRawWide wload_wide(const Chain &ch, int b, int half) {
+    WRawWide r;
+    const GAS uint8_t *u = ch.unit + (size_t)b * (TILE_ROWS * unit_bytes<DT_Q6_K>());
+#pragma unroll
+    for (int p = 0; p < 4; p++) r.ql[p] = *(const GAS u32x4 *)(u + 32 * p + 16 * half);
+#pragma unroll
+    for (int p = 0; p < 2; p++) r.qh[p] = *(const GAS u32x4 *)(u + 128 + 32 * p + 16 * half);
+    r.sc = *(const GAS u32x4 *)(u + 192);
+    r.d = ch.dp[b * TILE_ROWS];
+    return r;
+}
+
+/* thread (token j = tid / 4, part p = tid % 4) stages 64 code bytes; x in the split layout */
+struct StageWide {
+    u32x4 c[4];
+    float d;
+};
+__device__ __forceinline__ StageWide stage_wide_load(const GAS uint8_t *x, int nb, int b, int p) {
+    StageWide r;
+#pragma unroll
+    for (int k = 0; k < 4; k++) r.c[k] = *(const GAS u32x4 *)(x + (size_t)b * 256 + 16 * (4 * k + p));
+    r.d = *(const GAS float *)(x + (size_t)nb * 288 + 4 * b);
+    return r;
+}
+__device__ __forceinline__ void stage_wide_store(LAS uint8_t *buf, const StageWide &r, int j, int p) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) *(LAS u32x4 *)(buf + j * Wide::CS + 16 * (4 * k + p)) = r.c[k];
+    if (p == 0) *(LAS float *)(buf + Wide::D + 4 * j) = r.d;
+}
+
+/* one block against the tile's two 32-token halves; acc[16 i + v]: token 32 i + (v's token) */
+__device__ __forceinline__ void block_wide(const WRawWide &w, const LAS uint8_t *buf, int t, int half,
+                                           float (&acc)[32]) {
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    const LAS uint8_t *cod = buf + t * Wide::CS + 16 * half;
+    constexpr int NT = Wide::TOK / 32;
+    v16i H[NT], L[NT];
+#pragma unroll
+    for (int i = 0; i < NT; i++) H[i] = L[i] = v16i{};
+#pragma unroll
+    for (int s = 0; s < 8; s++) {   /* values 32 s .. 32 s + 31; the lane's 16 are group 2 s + half */
+        const int h = s >> 2, qq = s & 3, n4 = 4 * (qq >> 1), sh = 2 * qq;
+        const int sg = (int)(int8_t)((w.sc[s >> 1] >> (16 * (s & 1) + 8 * half)) & 0xFF);
+        const u16x2 sc2 = (unsigned short)sg, c2 = (unsigned short)(128 - 32 * sg);
+        v4i hi, lo;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t a = w.ql[2 * h + (qq & 1)][k], c = w.qh[h][k];
+            /* codes of bytes 0, 2 and of bytes 1, 3 in 16-bit halves */
+            const uint32_t ev = ((a >> n4) & 0x000F000Fu) | ((sh < 4 ? c << (4 - sh) : c >> (sh - 4)) & 0x00300030u);
+            const uint32_t od = ((a >> (n4 + 8)) & 0x000F000Fu) | ((c >> (sh + 4)) & 0x00300030u);
+            const uint32_t we = __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, ev) * sc2 + c2);   /* w + 128 */
+            const uint32_t wo = __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, od) * sc2 + c2);
+            hi[k] = (int)__builtin_amdgcn_perm(wo, we, 0x07030501u);
+            lo[k] = (int)(__builtin_amdgcn_perm(wo, we, 0x06020400u) ^ 0x80808080u);
+        }
+#pragma unroll
+        for (int i = 0; i < NT; i++) {
+            v4i ax = *(const LAS v4i *)(cod + 32 * i * Wide::CS + 32 * s);
+            H[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ax, hi, H[i], 0, 0, 0);
+            L[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ax, lo, L[i], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);   /* splitting several steps ahead would spill */
+    }
+    const float dw = f16_cvt(w.d);
+#pragma unroll
+    for (int i = 0; i < NT; i++) {
+        const LAS float *dd = (const LAS float *)(buf + Wide::D) + 32 * i + 4 * half;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const f32x4 da = *(const LAS f32x4 *)(dd + 8 * q);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int v = 4 * q + k;
+                acc[16 * i + v] = fmaf(dw * da[k], (float)((H[i][v] << 8) + L[i][v]), acc[16 * i + v]);
+            }
+        }
+    }
+}
+
+/* the group's tile, as tile_run: x: the activation of
+ * token tid / 4 (threads past the last token pass the last one's), lds:
+ * wide_lds_bytes() bytes; acc[16 i + v] = the row . token 32 i + 8 (v / 4) +
+ * 4 (l / 32) + v % 4 */
+__device__ __forceinline__ void tile_run_wide(const Chain &ch, int nb, const GAS uint8_t *x, LAS uint8_t *lds,
+                                              float (&acc)[32]) {
+    const int tid = threadIdx.x, j = tid >> 2, p = tid & 3, lane = tid & 63, t = lane & 31, half = lane >> 5;
+#pragma unroll
+    for (int v = 0; v < 32; v++) acc[v] = 0.0f;
+    StageWide r = stage_wide_load(x, nb, 0, p);
+    WRawWide w = wload_wide(ch, 0, half);
+    stage_wide_store(lds, r, j, p);
+    __syncthreads();
+    for (int b = 0; b < nb; b++) {
+        LAS uint8_t *cur = lds + (b & 1) * Wide::BYTES, *nxt = lds + (~b & 1) * Wide::BYTES;
+        const int bn = b + 1 < nb ? b + 1 : b;
+        WRawWide wn = wload_wide(ch, bn, half);
+        r = stage_wide_load(x, nb, bn, p);
+        block_wide(w, cur, t, half, acc);
+        stage_wide_store(nxt, r, j, p);
+        __syncthreads();
+        w = wn;
+    }
+}
+
 }  // namespace tokmm
 
 #endif
