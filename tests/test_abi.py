@@ -133,13 +133,12 @@ def test_host_checks_reject_bad_arguments_without_launching():
     assert lib.tlm_hip_quantize_act(15, None, 0, None, None) == 0     # n <= 0 is a no-op
 
 
-def _device_symbols(so_bytes):
-    """Global symbol names of every gfx950 code object in the library's
-    offload bundles (format: magic, entry count, then per entry offset, size,
-    triple length and triple; each entry an ELF64 code object)."""
+def _code_objects(so_bytes):
+    """The gfx950 code objects (ELF64) of the library's offload bundles
+    (format: magic, entry count, then per entry offset, size, triple length
+    and triple)."""
     import struct
     magic = b"__CLANG_OFFLOAD_BUNDLE__"
-    names, n_objs = set(), 0
     at = so_bytes.find(magic)
     while at >= 0:
         (n,) = struct.unpack_from("<Q", so_bytes, at + 24)
@@ -152,21 +151,29 @@ def _device_symbols(so_bytes):
                 continue
             elf = so_bytes[at + off:at + off + size]
             assert elf[:4] == b"\x7fELF", triple
-            n_objs += 1
-            shoff, = struct.unpack_from("<Q", elf, 0x28)
-            shentsize, shnum = struct.unpack_from("<HH", elf, 0x3A)
-            secs = [struct.unpack_from("<IIQQQQIIQQ", elf, shoff + i * shentsize) for i in range(shnum)]
-            for s in secs:
-                if s[1] != 2:   # SHT_SYMTAB
-                    continue
-                strtab = secs[s[6]]
-                for j in range(s[5] // 24):
-                    st_name, st_info = struct.unpack_from("<IB", elf, s[4] + j * 24)
-                    if st_info >> 4 != 1:   # STB_GLOBAL
-                        continue
-                    end = elf.index(b"\0", strtab[4] + st_name)
-                    names.add(elf[strtab[4] + st_name:end].decode())
+            yield elf
         at = so_bytes.find(magic, at + 24)
+
+
+def _device_symbols(so_bytes):
+    """Global symbol names of every gfx950 code object, and their number."""
+    import struct
+    names, n_objs = set(), 0
+    for elf in _code_objects(so_bytes):
+        n_objs += 1
+        shoff, = struct.unpack_from("<Q", elf, 0x28)
+        shentsize, shnum = struct.unpack_from("<HH", elf, 0x3A)
+        secs = [struct.unpack_from("<IIQQQQIIQQ", elf, shoff + i * shentsize) for i in range(shnum)]
+        for s in secs:
+            if s[1] != 2:   # SHT_SYMTAB
+                continue
+            strtab = secs[s[6]]
+            for j in range(s[5] // 24):
+                st_name, st_info = struct.unpack_from("<IB", elf, s[4] + j * 24)
+                if st_info >> 4 != 1:   # STB_GLOBAL
+                    continue
+                end = elf.index(b"\0", strtab[4] + st_name)
+                names.add(elf[strtab[4] + st_name:end].decode())
     return names, n_objs
 
 
@@ -189,3 +196,27 @@ def test_registered_kernels_exist_in_code_objects():
     assert len(registered) > 100
     missing = sorted(registered - dev)
     assert not missing, missing[:5]
+
+
+def test_no_kernel_spills_vector_registers():
+    """No kernel of the library spills a vector register to memory (the
+    compiler's own count in each code object's metadata): a loop that the
+    compiler unrolls and hoists past the register file still gives the right
+    bits, only many times slower."""
+    so = os.path.join(ROOT, "tierlm_amd", "libtlm_hip.so")
+    if not os.path.exists(so):
+        pytest.skip("library not built")
+    spills = {}
+    with tempfile.TemporaryDirectory() as d:
+        for i, elf in enumerate(_code_objects(open(so, "rb").read())):
+            f = os.path.join(d, "%d.co" % i)
+            open(f, "wb").write(elf)
+            notes = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", f], capture_output=True, text=True,
+                                   check=True).stdout
+            for k in re.split(r"\n  - ", notes)[1:]:
+                name = re.search(r"\.symbol:\s+(\S+)", k)
+                count = re.search(r"\.vgpr_spill_count:\s+(\d+)", k)
+                if name and count:
+                    spills[name.group(1)] = int(count.group(1))
+    assert len(spills) > 100
+    assert {k: v for k, v in spills.items() if v} == {}
