@@ -6,10 +6,12 @@
  *
  * Checked: the device activation quantisers (bytes), the plain-layout matvec
  * and the packed-layout matvec (bits of every row) for F32, Q8_0, Q4_K, Q5_K,
- * Q6_K and Q8_K, and the exponential against this host's libm expf.  Returns
- * the number of failing kernels; bit dt of *mask is set for every dtype whose
- * kernels failed, bit 30 for the exponential. */
+ * Q6_K and Q8_K, the exponential against this host's libm expf, and the
+ * matrix cores' float products against v_mul_f32.  Returns the number of
+ * failing kernels; bit dt of *mask is set for every dtype whose kernels failed,
+ * bit 30 for the exponential, bit 29 for the products. */
 #include "tlm_hip_internal.h"
+#include "tlm_hip_outer.h"
 
 #include <math.h>
 #include <stdlib.h>
@@ -194,6 +196,55 @@ bool same(float a, float b) {
     return x == y;
 }
 
+/* bad[64 g + l]: whether one of lane l's products of group g (ROWS values of a,
+ * 64 of b) is not v_mul_f32's: the same value or both a NaN (a zero's sign is
+ * not compared, tlm_hip_outer.h) */
+template <int ROWS>
+__global__ __launch_bounds__(64) void k_outer_check(const float *__restrict__ a, const float *__restrict__ b,
+                                                    uint32_t *__restrict__ bad) {
+    using O = Outer<ROWS>;
+    const int lane = threadIdx.x;
+    a += ROWS * blockIdx.x;
+    b += 64 * blockIdx.x;
+    const typename O::T p = O::mul(a[lane % ROWS], b[lane]);
+    uint32_t diff = 0;
+#pragma unroll
+    for (int v = 0; v < ROWS; v++) {
+        const float want = a[O::row(v, lane)] * b[O::col(v, lane)], got = p[v];
+        if (want != got && !(want != want && got != got)) diff = 1;
+    }
+    bad[64 * blockIdx.x + lane] = diff;
+}
+
+/* every shape over pairs of the values where a product rounds, overflows or
+ * vanishes, and over random bit patterns; dev: 64 KB */
+bool outer_ok(uint8_t *dev, uint32_t *s) {
+    const int G = 64;
+    static const uint32_t edge[16] = {0x00000000u, 0x00000001u, 0x00000003u, 0x00400001u, 0x007FFFFFu, 0x00800000u,
+                                      0x00800001u, 0x1F800000u, 0x20000001u, 0x3F000000u, 0x3F7FFFFFu, 0x3F800001u,
+                                      0x40400000u, 0x7F7FFFFFu, 0x7F800000u, 0x7FC00000u};
+    std::vector<uint32_t> a(32 * G), b(64 * G), bad(64 * G);
+    for (int i = 0; i < 32 * G; i++)   /* the first half: every edge with both signs */
+        a[i] = i < 16 * G ? edge[i & 15] | (uint32_t)(i >> 4 & 1) << 31 : st_rng(s) << 16 ^ st_rng(s);
+    for (int i = 0; i < 64 * G; i++)
+        b[i] = i < 32 * G ? edge[(i + i / 64) & 15] | (uint32_t)(i >> 5 & 1) << 31 : st_rng(s) << 16 ^ st_rng(s);
+    float *da = (float *)dev, *db = (float *)(dev + 16384);
+    uint32_t *dbad = (uint32_t *)(dev + 32768);
+    if (hipMemcpy(da, a.data(), a.size() * 4, hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(db, b.data(), b.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
+        return false;
+    bool ok = true;
+    for (int rows : {32, 16, 4}) {
+        if (rows == 32) hipLaunchKernelGGL(k_outer_check<32>, dim3(G), dim3(64), 0, nullptr, da, db, dbad);
+        else if (rows == 16) hipLaunchKernelGGL(k_outer_check<16>, dim3(G), dim3(64), 0, nullptr, da, db, dbad);
+        else hipLaunchKernelGGL(k_outer_check<4>, dim3(G), dim3(64), 0, nullptr, da, db, dbad);
+        ok = ok && hipGetLastError() == hipSuccess &&
+             hipMemcpy(bad.data(), dbad, bad.size() * 4, hipMemcpyDeviceToHost) == hipSuccess;
+        for (size_t i = 0; ok && i < bad.size(); i++) ok = bad[i] == 0;
+    }
+    return ok;
+}
+
 }  // namespace
 
 int tlmh_selftest(int *failed_mask) {
@@ -286,6 +337,10 @@ int tlmh_selftest(int *failed_mask) {
             fails++;
             mask |= 1 << 30;
         }
+    }
+    if (!outer_ok(dev + o_p, &s)) {
+        fails++;
+        mask |= 1 << 29;
     }
     (void)hipDeviceSynchronize();
     (void)hipFree(dev);
