@@ -257,3 +257,15 @@ def test_attention_row_tiles(hip, heads, kv, hd):
     tokens of one tile at positions on both sides of a group's end."""
     compare_models(dict(BASE, n_heads=heads, n_kv_heads=kv, head_dim=hd), 14, 8, True, 0, [15, 1, 17, 31, 33, 2, 64],
                    n_after=2)
+
+
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+def test_attention_four_row_tiles(hip, hd):
+    """The attention launches' tiles of four rows (few rows) and their large
+    ones: chunks on both sides of a wave per SIMD, one row more than a tile,
+    contexts with 0 to 5 whole groups of 16 positions behind a prompt long
+    enough that every buffer of the four is used."""
+    compare_models(dict(BASE, n_heads=16, n_kv_heads=16, head_dim=hd), 14, 8, True, 0,
+                   [1, 15, 1, 17, 5, 47, 3, 64, 130, 2], n_after=2)
+    compare_models(dict(BASE, n_heads=8, n_kv_heads=2, head_dim=hd), 14, 8, True, 0, [80, 3, 600, 1], n_after=2,
+                   max_ctx=700)

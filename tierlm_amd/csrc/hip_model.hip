@@ -20,6 +20,7 @@
 #include "tlm_hip_internal.h"
 #include <hip/hip_fp16.h>
 #include "tlm_hip_act.h"
+#include "tlm_hip_outer.h"
 
 #include <math.h>
 #include <stdlib.h>
@@ -945,34 +946,41 @@ __global__ __launch_bounds__(NT) void k_attn_merge(const float *__restrict__ par
  * k_pf_prep: a group per token: q-norm + RoPE of every query head in place,
  *   k-norm + RoPE of every key head (norm_rope16, the decode's code), the key
  *   and value appended to the cache at the token's position.
- * k_pf_scores: a wave per (key head, PF_SROWS rows, 64 positions), a row being
- *   one query head of one token; each score is the dot in ascending i, scaled
+ * k_pf_scores: a wave per (key head, row tile, 64 positions), a row being one
+ *   query head of one token; each score is the dot in ascending i, scaled
  *   after the dot (the decode's expression).
  * k_pf_softmax: a group per (token, query head): the decode P.V launch's
  *   softmax with its thread mapping and reduction trees (the maximum, e_t,
  *   their double sum, inv); p_t = e_t * inv replaces the score.
- * k_pf_pv: a wave per (key head, 64-element slab, PF_VROWS rows), out +=
+ * k_pf_pv: a wave per (key head, 64-element slab, row tile), out +=
  *   p_t * v_t[i] over ascending t up to the row's position (the rounded
  *   product, then the add); a group's waves share their rows' probabilities.
  * The dots and P.V are chains of a rounded product and a rounded add, and an
  * fma would round once.  The products of one i (one t) over a tile are an
- * outer product: v_mfma_f32 with K = 1 and C = 0 gives each of them with the
- * rounding of v_mul_f32 (subnormals and signed zeros included), 2048 in 64
- * lanes, and the VALU only adds.  Operands come from L1 / L2 straight into
- * registers, 16 elements (positions) ahead of their use, so no LDS read sits
- * between the adds: with the products on the VALU and the query values or
- * probabilities broadcast from LDS both launches waited for LDS.  At 682
- * tokens behind 1365 positions, 32 heads of 128 (4.8 G products each): scores
- * 381 -> 211 us, P.V 387 -> 195 us (24.5 G products / ms; a loop of the two
- * instructions alone runs at 34.5, v_mul + v_add at 26.4).  Bound: VALU issue
- * of the adds and the matrix pipe, which do not fully overlap.  P.V takes 16
- * rows a wave (the score launch 32): its chains are as long as the context, so
- * waves are what is short.
+ * outer product from the matrix cores (tlm_hip_outer.h), 2048 in 64 lanes, and
+ * the VALU only adds.  Operands come from L1 / L2 straight into registers, 16
+ * elements (positions) ahead of their use, so no LDS read sits between the
+ * adds: with the products on the VALU and the query values or probabilities
+ * broadcast from LDS both launches waited for LDS.  At 682 tokens behind 1365
+ * positions, 32 heads of 128 (4.8 G products each): scores 381 -> 211 us, P.V
+ * 387 -> 195 us (24.5 G products / ms; a loop of the two instructions alone
+ * runs at 34.5, v_mul + v_add at 26.4).  Bound: VALU issue of the adds and the
+ * matrix pipe, which do not fully overlap.
+ * Row tiles: PF_SROWS (PF_VROWS: a P.V chain is as long as the context, so
+ * waves are what is short) for launches that fill the chip.  Where tiles of
+ * four rows give at most a wave per SIMD, what counts is one wave's chain, 64
+ * to 130 cycles an element in the large tiles for the products and adds of
+ * rows that may not exist, and about 24 in a tile of four, whose loads run 64
+ * ahead.  Measured, four-row tiles against the large ones (whole prompts, us):
+ * P.V of 16 tokens behind 2000 positions, four layers of 8 heads of 64: 919
+ * against 741 (32 waves), of 16 behind 2000, two layers of 32 heads of 128:
+ * 778, 678 (256 waves), of 80: 906, 889 (1280), of 200 with 16 key heads: 846,
+ * 889 (1600); scores at 128 waves 546, 521, at 1024 1013, 999, at 1280 729,
+ * 739, at 8192 752, 828.
  * Score rows: [token][query head][SL] floats, SL the capacity rounded up to 4. */
 constexpr int PF_SROWS = 32;  /* rows per wave of the score launch */
 constexpr int PF_VROWS = 16;  /* rows per wave of the P.V launch */
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v32f __attribute__((ext_vector_type(32)));
+constexpr int PF_SIMDS = 1024;
 __host__ __device__ constexpr int pf_slabs(int hd) { return (hd + 63) / 64; }
 
 template <int HD>
@@ -1013,22 +1021,23 @@ __global__ __launch_bounds__(NT) void k_pf_prep(float *__restrict__ q, const flo
 }
 
 /* the launch's rows of one key head: row r is query head r % R of token r / R */
-template <int HD>
+template <int HD, int ROWS>
 __global__ __launch_bounds__(NT) void k_pf_scores(const float *__restrict__ q, const float *__restrict__ kc,
                                                   float *__restrict__ scores, int H, int KV, int max_ctx, int p0,
                                                   int ntok, int SL) {
-    constexpr int NC = HD / 16;   /* chunks of 16 elements, an even number */
-    static_assert(HD % 32 == 0, "chunks go in pairs");
+    using O = Outer<ROWS>;
+    constexpr int NC = HD / 16, ST = ROWS > 4 ? 2 : NC % 4 == 0 ? 4 : NC % 3 == 0 ? 3 : 2;   /* chunks of 16 elements, buffers */
+    static_assert(NC % ST == 0, "chunks fill the buffers");
     const int R = H / KV, kvh = blockIdx.z, lane = threadIdx.x & 63, nrows = ntok * R;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r0 = ((int)blockIdx.y * (NT / 64) + wave) * PF_SROWS, u0 = (int)blockIdx.x * 64;
-    const int plast = p0 + min(r0 + PF_SROWS - 1, nrows - 1) / R;
+    const int r0 = ((int)blockIdx.y * (NT / 64) + wave) * ROWS, u0 = (int)blockIdx.x * 64;
+    const int plast = p0 + min(r0 + ROWS - 1, nrows - 1) / R;
     if (r0 >= nrows || u0 > plast) return;   /* uniform over the wave; the kernel has no barrier */
     /* rows past the launch's last and positions past the wave's last are clamped, never stored */
-    const int ra = min(r0 + (lane & 31), nrows - 1);
+    const int ra = min(r0 + lane % ROWS, nrows - 1);
     const f32x4 *A4 = (const f32x4 *)(q + ((size_t)(ra / R) * H + kvh * R + ra % R) * HD);
     const f32x4 *B4 = (const f32x4 *)(kc + ((size_t)kvh * max_ctx + min(u0 + lane, plast)) * HD);
-    f32x4 a[2][4], b[2][4];
+    f32x4 a[ST][4], b[ST][4];
     auto load = [&](int s, int c) {
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -1036,45 +1045,47 @@ __global__ __launch_bounds__(NT) void k_pf_scores(const float *__restrict__ q, c
             b[s][k] = B4[4 * c + k];
         }
     };
-    float acc[32];
+    float acc[ROWS];
 #pragma unroll
-    for (int v = 0; v < 32; v++) acc[v] = 0.0f;
-    load(0, 0);
-    v32f pr = __builtin_amdgcn_mfma_f32_32x32x1f32(a[0][0].x, b[0][0].x, v32f{}, 0, 0, 0);
-    /* a loop at every width: with the trip count known (one at 32, two at 64)
-     * it was unrolled into one block whose MFMAs, which wait for no add, were
-     * all hoisted: 704 and 1632 spilled registers, and 102.7 ms for a prompt
-     * of 2047 tokens through four layers of 8 heads of 64 that takes 2.4 */
+    for (int v = 0; v < ROWS; v++) acc[v] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < ST - 1; s++) load(s, s);
+    typename O::T pr = O::mul(a[0][0].x, b[0][0].x);
+    /* a loop at every width: with a trip count of one or two known (widths of
+     * 32 and 64) it was unrolled into one block whose MFMAs, which wait for no
+     * add, were all hoisted: 704 and 1632 spilled registers, and 102.7 ms for
+     * a prompt of 2047 tokens through four layers of 8 heads of 64 that takes
+     * 2.4 */
     int nc = NC;
-    asm("" : "+s"(nc));
+    if (NC <= 2 * ST) asm("" : "+s"(nc));
 #pragma unroll 1
-    for (int c = 0; c < nc; c += 2) {
+    for (int c = 0; c < nc; c += ST) {
 #pragma unroll
-        for (int s = 0; s < 2; s++) {
-            load(s ^ 1, min(c + s + 1, NC - 1));
+        for (int s = 0; s < ST; s++) {
+            load((s + ST - 1) % ST, min(c + s + ST - 1, NC - 1));
 #pragma unroll
             for (int e = 0; e < 16; e++) {   /* element e + 1's products are issued before element e's are added */
-                const f32x4 an = e < 15 ? a[s][(e + 1) >> 2] : a[s ^ 1][0];
-                const f32x4 bn = e < 15 ? b[s][(e + 1) >> 2] : b[s ^ 1][0];
-                const v32f nx = __builtin_amdgcn_mfma_f32_32x32x1f32(an[(e + 1) & 3], bn[(e + 1) & 3], v32f{}, 0, 0, 0);
+                const f32x4 an = e < 15 ? a[s][(e + 1) >> 2] : a[(s + 1) % ST][0];
+                const f32x4 bn = e < 15 ? b[s][(e + 1) >> 2] : b[(s + 1) % ST][0];
+                const typename O::T nx = O::mul(an[(e + 1) & 3], bn[(e + 1) & 3]);
 #pragma unroll
-                for (int v = 0; v < 32; v++) acc[v] += pr[v];
+                for (int v = 0; v < ROWS; v++) acc[v] += pr[v];
                 pr = nx;
-                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);    /* one MFMA, */
-                __builtin_amdgcn_sched_group_barrier(0x2, 32, 0);   /* then the adds */
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);      /* one MFMA, */
+                __builtin_amdgcn_sched_group_barrier(0x2, ROWS, 0);   /* then the adds */
             }
         }
     }
     const float scale = 1.0f / sqrtf((float)HD);
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const int r = r0 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3), t = r / R;
+    for (int v = 0; v < O::RV; v++) {
+        const int r = r0 + O::row(v, lane), t = r / R;
         if (r >= nrows) continue;
         float *S = scores + ((size_t)t * H + kvh * R + r % R) * SL;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int u = u0 + 32 * h + (lane & 31);
-            if (u <= p0 + t) S[u] = acc[16 * h + v] * scale;
+        for (int h = v; h < ROWS; h += O::RV) {
+            const int u = u0 + O::col(h, lane);
+            if (u <= p0 + t) S[u] = acc[h] * scale;
         }
     }
 }
@@ -1140,21 +1151,23 @@ __global__ __launch_bounds__(NT) void k_pf_softmax(float *__restrict__ scores, i
     }
 }
 
-template <int HD>
+template <int HD, int ROWS>
 __global__ __launch_bounds__(NT) void k_pf_pv(const float *__restrict__ scores, const float *__restrict__ vc,
                                               float *__restrict__ att, int H, int KV, int max_ctx, int p0, int ntok,
                                               int SL) {
+    using O = Outer<ROWS>;
     constexpr int NWC = pf_slabs(HD), RT = NT / 64 / NWC;   /* slabs, row tiles of a group */
+    constexpr int ST = ROWS > 4 ? 2 : 4;                    /* buffers of 16 positions */
     const int R = H / KV, kvh = blockIdx.x, lane = threadIdx.x & 63, nrows = ntok * R;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), slab = wave % NWC;
-    const int r0 = ((int)(gridDim.y - 1 - blockIdx.y) * RT + wave / NWC) * PF_VROWS;   /* the longest rows first */
+    const int r0 = ((int)(gridDim.y - 1 - blockIdx.y) * RT + wave / NWC) * ROWS;   /* the longest rows first */
     if (r0 >= nrows) return;   /* uniform over the wave; the kernel has no barrier */
-    const int ra = min(r0 + (lane & 15), nrows - 1);   /* rows past the last are clamped, never stored */
+    const int ra = min(r0 + lane % ROWS, nrows - 1);   /* rows past the last are clamped, never stored */
     const f32x4 *A4 = (const f32x4 *)(scores + ((size_t)(ra / R) * H + kvh * R + ra % R) * SL);
     const char *vbase = (const char *)(vc + (size_t)kvh * att_vstride(max_ctx, HD));
     const uint32_t lane_off = (uint32_t)min(64 * slab + lane, HD - 1) * 16u;   /* the element's 16 bytes of a tile */
     auto vtile = [&](int tq) { return *(const f32x4 *)(vbase + (size_t)tq * (HD * 16) + lane_off); };
-    f32x4 a[2][4], b[2][4];
+    f32x4 a[ST][4], b[ST][4];
     auto load = [&](int s, int g) {   /* positions 16 g .. 16 g + 15 */
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -1162,51 +1175,59 @@ __global__ __launch_bounds__(NT) void k_pf_pv(const float *__restrict__ scores, 
             b[s][k] = vtile(4 * g + k);
         }
     };
-    float acc[16];
+    float acc[ROWS];
 #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = 0.0f;
+    for (int v = 0; v < ROWS; v++) acc[v] = 0.0f;
     /* whole groups of 16 positions that every row of the tile attends to */
     const int ng = (p0 + r0 / R + 1) / 16;
     if (ng > 0) {
-        load(0, 0);
-        v16f pr = __builtin_amdgcn_mfma_f32_16x16x1f32(a[0][0].x, b[0][0].x, v16f{}, 0, 0, 0);
+#pragma unroll
+        for (int s = 0; s < ST - 1; s++) load(s, s ? min(s, ng - 1) : 0);
+        typename O::T pr = O::mul(a[0][0].x, b[0][0].x);
         auto group = [&](int s, int next) {
-            load(s ^ 1, min(next, ng - 1));
+            load((s + ST - 1) % ST, min(next, ng - 1));
 #pragma unroll
             for (int e = 0; e < 16; e++) {   /* position e + 1's products are issued before position e's are added */
-                const f32x4 an = e < 15 ? a[s][(e + 1) >> 2] : a[s ^ 1][0];
-                const f32x4 bn = e < 15 ? b[s][(e + 1) >> 2] : b[s ^ 1][0];
-                const v16f nx = __builtin_amdgcn_mfma_f32_16x16x1f32(an[(e + 1) & 3], bn[(e + 1) & 3], v16f{}, 0, 0, 0);
+                const f32x4 an = e < 15 ? a[s][(e + 1) >> 2] : a[(s + 1) % ST][0];
+                const f32x4 bn = e < 15 ? b[s][(e + 1) >> 2] : b[(s + 1) % ST][0];
+                const typename O::T nx = O::mul(an[(e + 1) & 3], bn[(e + 1) & 3]);
 #pragma unroll
-                for (int v = 0; v < 16; v++) acc[v] += pr[v];
+                for (int v = 0; v < ROWS; v++) acc[v] += pr[v];
                 pr = nx;
-                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);    /* one MFMA, */
-                __builtin_amdgcn_sched_group_barrier(0x2, 16, 0);   /* then the adds */
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);      /* one MFMA, */
+                __builtin_amdgcn_sched_group_barrier(0x2, ROWS, 0);   /* then the adds */
             }
         };
-        for (int g = 0; g < ng; g += 2) {
-            group(0, g + 1);
+        for (int g = 0; g < ng; g += ST) {
+            group(0, g + ST - 1);
             if (g + 1 >= ng) break;
-            group(1, g + 2);
+            group(1, g + ST);
+            if constexpr (ST == 4) {
+                if (g + 2 >= ng) break;
+                group(2, g + 5);
+                if (g + 3 >= ng) break;
+                group(3, g + 6);
+            }
         }
     }
     /* the rest: a product past its row's position is dropped, not added (0 * inf would not be 0) */
+    static_assert(O::RV == 4, "rows of P");
     int P[4];
 #pragma unroll
-    for (int k = 0; k < 4; k++) P[k] = p0 + (r0 + 4 * (lane >> 4) + k) / R;
-    const int pmax = p0 + min(r0 + PF_VROWS - 1, nrows - 1) / R;
+    for (int k = 0; k < 4; k++) P[k] = p0 + (r0 + O::row(k, lane)) / R;
+    const int pmax = p0 + min(r0 + ROWS - 1, nrows - 1) / R;
     for (int u = 16 * ng; u <= pmax; u += 4) {
         const f32x4 at = A4[u >> 2], vt = vtile(u >> 2);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const v16f pr = __builtin_amdgcn_mfma_f32_16x16x1f32(at[e], vt[e], v16f{}, 0, 0, 0);
+            const typename O::T pr = O::mul(at[e], vt[e]);
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[v] = u + e <= P[v & 3] ? acc[v] + pr[v] : acc[v];
+            for (int v = 0; v < ROWS; v++) acc[v] = u + e <= P[v & 3] ? acc[v] + pr[v] : acc[v];
         }
     }
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const int r = r0 + 4 * (lane >> 4) + (v & 3), ic = 64 * slab + 16 * (v >> 2) + (lane & 15);
+    for (int v = 0; v < ROWS; v++) {
+        const int r = r0 + O::row(v, lane), ic = 64 * slab + O::col(v, lane);
         if (r < nrows && ic < HD) att[((size_t)(r / R) * H + kvh * R + r % R) * HD + ic] = acc[v];
     }
 }
@@ -1215,36 +1236,6 @@ __global__ __launch_bounds__(NT) void k_pf_pv(const float *__restrict__ scores, 
  * registers: head width at most 128) */
 bool pf_att_supported(int hd, int H, int KV) {
     return (hd == 32 || hd == 64 || hd == 96 || hd == 128) && KV > 0 && H % KV == 0;
-}
-
-/* the four prefill attention launches for ntok tokens at p0 (q rotated in
- * place, K/V appended, att [ntok][H][hd]) */
-int launch_pf_attn(int hd, int H, int KV, int max_ctx, int p0, int ntok, float *q, const float *kx, const float *vx,
-                   const float *q_norm, const float *k_norm, const float *cs, const float *sn, float *kc, float *vc,
-                   float *scores, int SL, float *att, float eps, hipStream_t s) {
-    const int has_qn = q_norm != nullptr, has_kn = k_norm != nullptr;
-    if (!q_norm) q_norm = q;   /* read and dropped */
-    if (!k_norm) k_norm = q;
-    const int rows = ntok * (H / KV);   /* of one key head */
-    const int rs = NT / 64 * PF_SROWS, rv = NT / 64 / pf_slabs(hd) * PF_VROWS;
-    const dim3 gsc((unsigned)((p0 + ntok + 63) / 64), (unsigned)((rows + rs - 1) / rs), (unsigned)KV);
-    const dim3 gpv((unsigned)KV, (unsigned)((rows + rv - 1) / rv));
-#define TLM_PF(W)                                                                                                \
-    case W:                                                                                                      \
-        hipLaunchKernelGGL((k_pf_prep<W>), dim3((unsigned)ntok), dim3(NT), 0, s, q, kx, vx, q_norm, k_norm,     \
-                           has_qn, has_kn, cs, sn, kc, vc, H, KV, max_ctx, p0, eps);                            \
-        hipLaunchKernelGGL((k_pf_scores<W>), gsc, dim3(NT), 0, s, (const float *)q, (const float *)kc, scores,  \
-                           H, KV, max_ctx, p0, ntok, SL);                                                       \
-        hipLaunchKernelGGL(k_pf_softmax, dim3((unsigned)H, (unsigned)ntok), dim3(NT), 0, s, scores, H, p0, SL); \
-        hipLaunchKernelGGL((k_pf_pv<W>), gpv, dim3(NT), 0, s, (const float *)scores, (const float *)vc, att, H, \
-                           KV, max_ctx, p0, ntok, SL);                                                          \
-        break;
-    switch (hd) {
-        TLM_PF(32) TLM_PF(64) TLM_PF(96) TLM_PF(128)
-    default: return tlmh_seterr(TLM_HIP_EUNSUP, "model prefill: head width %d", hd);
-    }
-#undef TLM_PF
-    return tlmh_check(hipGetLastError(), "model: prefill attention");
 }
 
 /* slices per key head: enough groups to cover the chip at long contexts
@@ -1301,6 +1292,39 @@ int launch_attn(int hd, int H, int KV, int max_ctx, int G, bool split, const flo
     }
 #undef TLM_ATT
     return tlmh_check(hipGetLastError(), "model: attention");
+}
+
+/* the four prefill attention launches for ntok tokens at p0 (q rotated in
+ * place, K/V appended, att [ntok][H][hd]) */
+int launch_pf_attn(int hd, int H, int KV, int max_ctx, int p0, int ntok, float *q, const float *kx, const float *vx,
+                   const float *q_norm, const float *k_norm, const float *cs, const float *sn, float *kc, float *vc,
+                   float *scores, int SL, float *att, float eps, hipStream_t s) {
+    const int has_qn = q_norm != nullptr, has_kn = k_norm != nullptr;
+    if (!q_norm) q_norm = q;   /* read and dropped */
+    if (!k_norm) k_norm = q;
+    const int rows = ntok * (H / KV);   /* of one key head */
+    const int nw = NT / 64, pt = (p0 + ntok + 63) / 64, slabs = pf_slabs(hd);
+    const int64_t tiles4 = (int64_t)KV * ((rows + 3) / 4);
+    const bool s4 = tiles4 * pt <= PF_SIMDS, v4 = tiles4 * slabs <= PF_SIMDS;
+    const int rs = nw * (s4 ? 4 : PF_SROWS), rv = nw / slabs * (v4 ? 4 : PF_VROWS);
+    const dim3 gsc((unsigned)pt, (unsigned)((rows + rs - 1) / rs), (unsigned)KV);
+    const dim3 gpv((unsigned)KV, (unsigned)((rows + rv - 1) / rv));
+#define TLM_PF(W)                                                                                                \
+    case W:                                                                                                      \
+        hipLaunchKernelGGL((k_pf_prep<W>), dim3((unsigned)ntok), dim3(NT), 0, s, q, kx, vx, q_norm, k_norm,     \
+                           has_qn, has_kn, cs, sn, kc, vc, H, KV, max_ctx, p0, eps);                            \
+        hipLaunchKernelGGL((s4 ? k_pf_scores<W, 4> : k_pf_scores<W, PF_SROWS>), gsc, dim3(NT), 0, s,            \
+                           (const float *)q, (const float *)kc, scores, H, KV, max_ctx, p0, ntok, SL);          \
+        hipLaunchKernelGGL(k_pf_softmax, dim3((unsigned)H, (unsigned)ntok), dim3(NT), 0, s, scores, H, p0, SL); \
+        hipLaunchKernelGGL((v4 ? k_pf_pv<W, 4> : k_pf_pv<W, PF_VROWS>), gpv, dim3(NT), 0, s,                    \
+                           (const float *)scores, (const float *)vc, att, H, KV, max_ctx, p0, ntok, SL);        \
+        break;
+    switch (hd) {
+        TLM_PF(32) TLM_PF(64) TLM_PF(96) TLM_PF(128)
+    default: return tlmh_seterr(TLM_HIP_EUNSUP, "model prefill: head width %d", hd);
+    }
+#undef TLM_PF
+    return tlmh_check(hipGetLastError(), "model: prefill attention");
 }
 
 /* end of a step: with the lm_head tiles' greedy keys (argmax_key of their
