@@ -271,6 +271,28 @@ def test_cached_prompt_batched_matches_resident(hip, edt, shared, budget, chunk)
         c.close()
 
 
+@pytest.mark.parametrize("budget", [TINY, 12 * 3 * 256 * 512 // 256 * 210])
+def test_cached_prompt_wide_expert_tiles(hip, budget):
+    """250 tokens x top-4 over 32 Q6_K experts: a mean past 30 slots, so
+    64-slot tiles, in passes that skip the experts of the other passes; the
+    resident batched prompt's and the cached step-by-step prompt's bits."""
+    from tierlm_amd.model import Model, bench_prompt
+    a = Model.synth(SMALL, expert_dt=14, seed=6, max_ctx=260)
+    b = Model.synth(SMALL, expert_dt=14, seed=6, max_ctx=260, expert_cache=budget)
+    c = Model.synth(SMALL, expert_dt=14, seed=6, max_ctx=260, expert_cache=budget, prefill_chunk=-1)
+    try:
+        assert a.prefill_batched() and b.prefill_batched() and not c.prefill_batched()
+        p = bench_prompt(250, SMALL["vocab"], seed=5)
+        la, lb, lc = a.prefill(p), b.prefill(p), c.prefill(p)
+        assert np.array_equal(la.view(np.uint32), lb.view(np.uint32))
+        assert np.array_equal(lc.view(np.uint32), lb.view(np.uint32))
+        assert b.store_stats()["evictions"] > 0
+    finally:
+        a.close()
+        b.close()
+        c.close()
+
+
 @needs_c3s
 def test_c3s_cached_batched_prefill_reference_bits(hip):
     """Qwen3-30B-A3B attention geometry, 16 experts top-8 through 8 slots,

@@ -13,7 +13,8 @@ import pytest
 import torch
 
 import oracle
-from tests.synth import build_moe_case
+from tests.synth import build_moe_case, device_block
+from tests.test_hip_gemv import same
 
 pytestmark = pytest.mark.gpu
 
@@ -153,7 +154,48 @@ def test_prefill_rejects_unsupported(hip, dev):
                                         (2, 2, 64, 512, 256), (3, 2, 97, 768, 256), (2, 1, 131, 256, 256)])
 def test_prefill_wide_tiles(hip, dev, E, k, T, D, de):
     """Q6_K experts around the mean of slots per expert where tiles take 64
-    slots (59 tokens: below, 60: at it), tiles of 33, 64 and one slot, an odd
-    number of blocks, against the decode block per token."""
+    slots (59 tokens: below, 60: at it), tiles of 33, 64 and a few slots, an
+    odd number of blocks, against the decode block per token."""
     case = build_moe_case(D=D, de=de, E=E, k=k, expert_dt=oracle.Q6_K, seed=T, device=dev)
     prefill_vs_decode(case, dev, T, seed=T + 1)
+
+
+@pytest.mark.parametrize("poison", [False, True])
+def test_prefill_wide_tile_edges(hip, dev, poison):
+    """Both of two experts for every one of 65 tokens: 64-slot tiles that are
+    full and of one slot.  Weight rows at the ends of the scaled planes (codes
+    0 and 63 under scales of -128 and 127: products of 4096, -3968, -4064 and
+    3937); with poison also tokens of zeros, with a NaN, with an infinity and
+    past the range of the rmsnorm's square, one of them alone in its tile."""
+    D, de, T = 512, 256, 65
+    case = build_moe_case(D=D, de=de, E=2, k=2, expert_dt=oracle.Q6_K, seed=31, weights="random_codes")
+    for mats in case.experts:
+        for W in mats:
+            blk = W.reshape(W.shape[0], -1, 210)
+            for r, (code, sc) in enumerate([(0x00, 0x80), (0xFF, 0x80), (0x00, 0x7F), (0xFF, 0x7F)]):
+                blk[r::5, :, 0:192] = code
+                blk[r::5, :, 192:208] = sc
+    case.block, case.dev_keep = device_block(case, dev)
+    rng = np.random.default_rng(32)
+    H = rng.standard_normal((T, D)).astype(np.float32)
+    if poison:
+        H[1] = 0.0
+        H[2, 5] = np.nan
+        H[3, D - 1] = np.inf
+        H[40] *= 1e30
+        H[T - 1, 300] = -np.inf
+    h = torch.from_numpy(H.copy()).to(dev)
+    ids = torch.empty((T, 2), dtype=torch.int32, device=dev)
+    w = torch.empty((T, 2), dtype=torch.float32, device=dev)
+    case.block.prefill(h, ids, w)
+    torch.cuda.synchronize()
+    got, got_ids, got_w = h.cpu().numpy(), ids.cpu().numpy(), w.cpu().numpy()
+    assert np.array_equal(np.bincount(got_ids.ravel(), minlength=2), [T, T])
+    for t in range(T):
+        ht = torch.from_numpy(H[t].copy()).to(dev)
+        case.block(ht)
+        torch.cuda.synchronize()
+        assert np.array_equal(got_ids[t], case.block.ids.cpu().numpy()[:2]), t
+        assert same(got_w[t], case.block.w.cpu().numpy()[:2]).all(), t
+        assert same(got[t], ht.cpu().numpy()).all(), f"token {t}"
+    assert np.isnan(got).any() == poison
