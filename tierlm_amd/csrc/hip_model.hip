@@ -968,10 +968,9 @@ __global__ __launch_bounds__(NT) void k_attn_merge(const float *__restrict__ par
  * matrix pipe, which do not fully overlap.
  * Row tiles: PF_SROWS (PF_VROWS: a P.V chain is as long as the context, so
  * waves are what is short) for launches that fill the chip.  Where tiles of
- * four rows give at most a wave per SIMD, what counts is one wave's chain, 64
- * to 130 cycles an element in the large tiles for the products and adds of
- * rows that may not exist, and about 24 in a tile of four, whose loads run 64
- * ahead.  Measured, four-row tiles against the large ones (whole prompts, us):
+ * four rows give at most a wave per SIMD, what counts is one wave's chain: a
+ * position of P.V takes 54 ns in a tile of 16 rows, most of which may not exist,
+ * and 24 to 31 in one of four, whose loads run 64 ahead.  Measured, four-row tiles against the large ones (whole prompts, us):
  * P.V of 16 tokens behind 2000 positions, four layers of 8 heads of 64: 919
  * against 741 (32 waves), of 16 behind 2000, two layers of 32 heads of 128:
  * 778, 678 (256 waves), of 80: 906, 889 (1280), of 200 with 16 key heads: 846,

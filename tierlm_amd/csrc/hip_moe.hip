@@ -956,9 +956,14 @@ struct PfLayout {
 /* Slots per tile: 64 for Q6_K once the experts average PF_WIDE_MEAN slots
  * (the wide tile: one pass over an expert's weights for up to 64 tokens, its
  * scales applied once), else 32: below that most experts fit one 32-slot tile,
- * which leaves three waves a SIMD instead of two.  128 experts of 768 x 2048,
- * top 8, gate/up + down: 512 tokens (mean 32) 192 -> 174 us, a prompt's chunks
- * of 682 (mean 43) 191 -> 154 us. */
+ * which leaves three waves a SIMD instead of two.  Whole blocks with 32- and
+ * with 64-slot tiles, us (uniform routing): 128 experts of 768 x 2048, top 8, at
+ * a mean of 15 slots 174, 196; 24: 200, 211; 28: 217, 217; 30: 227, 220; 32: 240,
+ * 222; 43: 302, 244; 64: 375, 333.  128 of 1536 x 4096: 15: 526, 637; 24: 575,
+ * 666; 30: 673, 685; 32: 719, 687.  32 of 256 x 512 (and a shared expert), top 4,
+ * whose grids leave compute units idle in both: 24: 61.9, 62.2; 30: 62.3, 62.9;
+ * 37: 65.8, 65.4; 64: 72.6, 70.7; 128: 88.3, 87.9.  The lines cross between 28
+ * and 34; the number of groups does not move them. */
 constexpr int PF_WIDE_MEAN = 30;
 inline int pf_tile_slots(const tlm_hip_moe_desc &d, int64_t T) {
     return d.expert_dt == DT_Q6_K && T * d.k >= (int64_t)PF_WIDE_MEAN * d.E ? tokmm::Wide::TOK : tokmm::TM_TOK;

@@ -6,7 +6,8 @@
  * the decode dot's bits: per super-block an exact int32 sum, then the row's
  * fma chain in ascending block order (src/lib/tlm_quant.c:812-882).
  *
- * A group of 4 waves streams its weight rows once for 32 tokens.  The
+ * A group of 4 waves streams its weight rows once for 32 tokens (Q6_K experts
+ * with enough of them: 64, tile_run_wide below).  The
  * tokens' Q8_K block is staged once in LDS for all 4 waves (two buffers, one
  * barrier per block); each wave streams 32 rows, with the weights and
  * activations of block b+1 in flight while block b computes.
