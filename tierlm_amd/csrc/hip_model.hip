@@ -970,7 +970,7 @@ __global__ __launch_bounds__(NT) void k_attn_merge(const float *__restrict__ par
  * waves are what is short) for launches that fill the chip.  Where tiles of
  * four rows give at most a wave per SIMD, what counts is one wave's chain: a
  * position of P.V takes 54 ns in a tile of 16 rows, most of which may not exist,
- * and 24 to 31 in one of four, whose loads run 64 ahead.  Measured, four-row tiles against the large ones (whole prompts, us):
+ * and 24 to 31 in one of four, whose loads run 48 ahead.  Measured, four-row tiles against the large ones (whole prompts, us):
  * P.V of 16 tokens behind 2000 positions, four layers of 8 heads of 64: 919
  * against 741 (32 waves), of 16 behind 2000, two layers of 32 heads of 128:
  * 778, 678 (256 waves), of 80: 906, 889 (1280), of 200 with 16 key heads: 846,
@@ -979,7 +979,7 @@ __global__ __launch_bounds__(NT) void k_attn_merge(const float *__restrict__ par
  * Score rows: [token][query head][SL] floats, SL the capacity rounded up to 4. */
 constexpr int PF_SROWS = 32;  /* rows per wave of the score launch */
 constexpr int PF_VROWS = 16;  /* rows per wave of the P.V launch */
-constexpr int PF_SIMDS = 1024;
+constexpr int PF_SIMDS = 1024;   /* 256 compute units of four */
 __host__ __device__ constexpr int pf_slabs(int hd) { return (hd + 63) / 64; }
 
 template <int HD>
